@@ -28,7 +28,7 @@
 extern "C" {
 #endif
 
-#define SGL_ABI_VERSION 22
+#define SGL_ABI_VERSION 23
 
 #define SGL_OK 0
 #define SGL_ERR_INVALID 1   /* bad argument (host-checked) */
@@ -435,6 +435,52 @@ int sgl_conv_backward(int32_t D, int32_t F, int32_t T, int32_t H,
                       float *sigma, float *gQ, float *ln_part, float *te_part,
                       float p_att, float p_out, uint64_t seed,
                       const uint64_t *rng_step, int32_t pass,
+                      const float *sv_sdrop, const sgl_bf16_weights *bw,
+                      hipStream_t stream);
+/* The same for `npass` (1 to 16) dropout passes pass, pass + 1, ... in one
+ * launch (one grid row a pass: a pass of a small batch leaves most of the GPU
+ * idle, and the passes do not depend on each other). The saved state arrays
+ * hold npass consecutive blocks of one pass's size, pass p's output starts at
+ * y + p * y_pass_stride. In the backward the gradient arrays and acc_src /
+ * g_src [npass][capacity+1][D] hold such blocks too, ln_part / te_part blocks
+ * of part_tiles tiles; acc_dst and gy are NULL, pass 0's dL/dy comes through
+ * w_s and every other pass's through w_d (the src, dst and negative roles of
+ * runtime.py:193-195). npass 1 is the single-pass call. */
+int sgl_conv_forward_passes(int32_t D, int32_t F, int32_t T, int32_t H,
+                     int32_t fanout, int64_t capacity,
+                     const int32_t *num_roots, const int32_t *any_edges,
+                     const float *h_root, const int32_t *cnt, float *X,
+                     const float *dt, const float *w_q, const float *b_q,
+                     const float *w_k, const float *b_k, const float *w_v,
+                     const float *b_v, const float *w_out, const float *b_out,
+                     const float *ln_g, const float *ln_b, const float *te_w,
+                     const float *te_b, float *sv_Q, float *sv_qt,
+                     float *sv_xbar, float *sv_score, float *sv_ml,
+                     float *sv_agg, float *sv_z, float *sv_stats,
+                     float *sv_phi0, float *S, float *y, int64_t y_pass_stride,
+                     float p_att, float p_out, uint64_t seed, const uint64_t *rng_step,
+                     int32_t pass, int32_t npass, float *sv_sdrop, const sgl_bf16_weights *bw,
+                     hipStream_t stream);
+int sgl_conv_backward_passes(int32_t D, int32_t F, int32_t T, int32_t H,
+                      int32_t fanout, int64_t capacity,
+                      const int32_t *num_roots, const int32_t *any_edges,
+                      const int32_t *cnt, const float *X, const float *S,
+                      const float *dt, const float *w_q, const float *b_q,
+                      const float *w_k, const float *b_k, const float *w_v,
+                      const float *b_v, const float *w_out, const float *b_out,
+                      const float *ln_g, const float *ln_b, const float *te_b,
+                      const float *sv_Q, const float *sv_qt,
+                      const float *sv_xbar, const float *sv_score,
+                      const float *sv_ml, const float *sv_agg,
+                      const float *sv_z, const float *sv_stats,
+                      const float *gy, int64_t *acc_src, int64_t *acc_dst,
+                      const float *w_s, const float *w_d,
+                      float *g_src, float *g_dst,
+                      float *gz, float *gagg, float *G,
+                      float *sigma, float *gQ, float *ln_part, float *te_part,
+                      int64_t part_tiles,
+                      float p_att, float p_out, uint64_t seed,
+                      const uint64_t *rng_step, int32_t pass, int32_t npass,
                       const float *sv_sdrop, const sgl_bf16_weights *bw,
                       hipStream_t stream);
 /* The attention's dropout masks for rows [0, rows) of a pass, as the

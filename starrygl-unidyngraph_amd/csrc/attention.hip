@@ -34,6 +34,12 @@
 // are merged through LDS (global max, rescaled sums). The backward splits the
 // window the same way and sums the slices' gradient partials.
 //
+// Dropout passes (the three roles of a training step draw their own masks)
+// run as the rows of one grid: at 400 roots a pass is ~100 workgroups of one
+// CU each, so three launches in a row took three times as long as one (three
+// heads-of-2, 372-column passes, B = 200: forward 118 -> 41 us, backward
+// 108 -> 38 us a step).
+//
 // No 1/sqrt(d) scaling (models.py:125). The time-encoding argument is
 // fl(fl(dt * w) + b), then cos.
 #include <climits>
@@ -48,6 +54,7 @@ constexpr int kEC = 4;      // edges gathered per round trip
 constexpr int kMaxH = 4;
 constexpr int kMaxJ = 8;    // C <= 512
 constexpr int kMaxWaves = 16;
+constexpr int kMaxPasses = 16;  // dropout passes of one launch
 
 // Waves per workgroup for a (heads, column slots) instance: 16 (128 VGPRs
 // each) while the edge loop's per-lane [H][J] arrays fit, else 8 (256 VGPRs).
@@ -186,12 +193,12 @@ __global__ __launch_bounds__(kEdgeBlock) void k_edge_rows(
 
 // This lane's slice of edge row `row` (c = lane + 64*j; zero past C) with
 // its time-encoding columns computed from dt and the time encoding's
-// parameters (te_w / te_b, staged in LDS): cos into x and into the row,
-// sin into S's row.
+// parameters (te_w / te_b, staged in LDS): cos into x and (store) into the
+// row, sin into S's row.
 template <int JM>
 __device__ __forceinline__ void fill_row(const Dims &d, float *__restrict__ X, float *__restrict__ S, size_t row,
                                          const float *__restrict__ te_w, const float *__restrict__ te_b, float dtv,
-                                         int lane, float (&x)[JM]) {
+                                         int lane, bool store, float (&x)[JM]) {
 #pragma unroll
   for (int j = 0; j < JM; ++j) {
     const int c = lane + 64 * j;
@@ -202,8 +209,10 @@ __device__ __forceinline__ void fill_row(const Dims &d, float *__restrict__ X, f
       const int t = c - d.D - d.F;
       float sn;
       te_sincos(te_arg(dtv, te_w[t], te_b[t]), sn, v);
-      X[row * d.C + c] = v;
-      S[row * d.T + t] = sn;
+      if (store) {
+        X[row * d.C + c] = v;
+        S[row * d.T + t] = sn;
+      }
     }
     x[j] = v;
   }
@@ -260,6 +269,20 @@ struct ConvSaved {
   float *sdrop;  // [cap][H]     with attention dropout: sum of the kept, rescaled weights
 };
 
+// The saved state of dropout pass `pass`, the passes' blocks consecutive.
+__device__ __forceinline__ void to_pass(ConvSaved &sv, const Dims &d, size_t cap, int pass) {
+  const size_t rows = cap * pass;
+  sv.Q += rows * d.D;
+  sv.agg += rows * d.D;
+  sv.z += rows * d.D;
+  sv.qt += rows * d.H * d.C;
+  sv.xbar += rows * d.H * d.C;
+  if (sv.score != nullptr) sv.score += rows * d.k * d.H;
+  sv.ml += rows * d.H * 2;
+  sv.stats += rows * 2;
+  if (sv.sdrop != nullptr) sv.sdrop += rows * d.H;
+}
+
 struct FwdLds {
   int ldh, ldr, lda, ldq;
   float *HT;    // [16][ldh]  [h | cos(b)]
@@ -270,8 +293,8 @@ struct FwdLds {
   float *qb;    // [16][H]
   float *TW, *TB;  // [T] time-encoding weight / bias
   float *BK, *LG, *LB;  // [D] key bias, LayerNorm weight and bias (staged with the first loads)
-  float *part;  // [NW][H*C]  a slice's unnormalised sums (slices only)
-  float *pml;   // [NW][H][3] a slice's running max, sum and kept sum (slices only)
+  float *part;  // [slices][H*C]  a slice's unnormalised sums (slices of all roots; none with one slice a root)
+  float *pml;   // [slices][H][3] a slice's running max, sum and kept sum
   float *scr;   // [NW][4][64] partial sums of the four-row products (4-root tiles only)
   float *DT;    // [rows][k] the tile's edges' dt (16-wave instances: stage_dt)
   float *Ts;    // [ts_rows][T] the tile's edges' time encodings (cos), when staged
@@ -285,7 +308,8 @@ struct FwdLds {
 // earlier stores: loads and stores share one in-order counter).
 __host__ __device__ constexpr bool stage_dt(int nw, int rows) { return nw == 16 && rows > 0; }
 
-__host__ __device__ inline FwdLds fwd_lds(const Dims &d, float *base, int nw, int rows, bool slices) {
+// slices: window slices of the tile's roots together (0: one slice a root, nothing to merge)
+__host__ __device__ inline FwdLds fwd_lds(const Dims &d, float *base, int nw, int rows, int slices) {
   FwdLds L;
   L.ldh = sgl::lds_ld(d.D + d.T);
   L.ldr = sgl::lds_ld(d.D);
@@ -303,8 +327,8 @@ __host__ __device__ inline FwdLds fwd_lds(const Dims &d, float *base, int nw, in
   L.LG = L.BK + d.D;
   L.LB = L.LG + d.D;
   L.part = L.LB + d.D;
-  L.pml = L.part + (slices ? nw * d.H * d.C : 0);
-  L.scr = L.pml + (slices ? ((nw * d.H * 3 + 3) & ~3) : 0);
+  L.pml = L.part + slices * d.H * d.C;
+  L.scr = L.pml + ((slices * d.H * 3 + 3) & ~3);
   L.DT = L.scr + (rows == 4 ? nw * 256 : 0);
   L.Ts = L.DT + (stage_dt(nw, rows) ? ((rows * d.k + 3) & ~3) : 0);
   return L;
@@ -312,7 +336,7 @@ __host__ __device__ inline FwdLds fwd_lds(const Dims &d, float *base, int nw, in
 
 // ts_rows: edges whose time encodings are staged in LDS (roots per tile *
 // fanout), 0 = computed in the edge loop instead.
-inline size_t fwd_lds_floats(const Dims &d, int nw, int rows, bool slices, int ts_rows) {
+inline size_t fwd_lds_floats(const Dims &d, int nw, int rows, int slices, int ts_rows) {
   float *base = reinterpret_cast<float *>(uintptr_t(4096));
   const FwdLds L = fwd_lds(d, base, nw, rows, slices);
   return size_t(L.Ts + size_t(ts_rows) * d.T - base);
@@ -327,17 +351,17 @@ __global__ __launch_bounds__(NW * 64) void k_conv_fwd(
     Dims d, const int32_t *__restrict__ num_roots, const int32_t *__restrict__ any_edges,
     const float *__restrict__ h_root, const int32_t *__restrict__ cnt, float *__restrict__ X,
     const float *__restrict__ dt, float *__restrict__ S, ConvParams p, ConvSaved sv, float *__restrict__ y,
-    int ts_rows, sgl::DropCfg dc, sgl_bf16_weights bw) {
+    int64_t y_pass_stride, int ts_rows, sgl::DropCfg dc, sgl_bf16_weights bw) {
   constexpr int kWaves = NW, kBlock = NW * 64;
   constexpr int WPR = NW / RPW;  // waves per root in the edge phase
   constexpr int NS = WPR / HG;   // window slices per root (merged through LDS when > 1)
   constexpr int HL = HM / HG;    // heads per wave in the edge phase
   static_assert(RPW <= kRows && NW % RPW == 0, "tile shape");
-  static_assert(WPR % HG == 0 && HM % HG == 0 && (HG == 1 || NS == 1), "head groups");
+  static_assert(WPR % HG == 0 && HM % HG == 0, "head groups");
   static_assert(!(BF && DROP), "the bf16 products run without dropout");
   extern __shared__ __align__(16) float lds[];
   const int D = d.D, T = d.T, H = d.H, C = d.C, dh = d.dh, K = d.k;
-  const FwdLds L = fwd_lds(d, lds, NW, RPW, NS > 1);
+  const FwdLds L = fwd_lds(d, lds, NW, RPW, NS > 1 ? RPW * NS : 0);
   __shared__ int s_cnt[kRows];
   __shared__ float s_sd[kRows][kMaxH];  // with attention dropout: the rows' kept-weight sums
 
@@ -348,6 +372,11 @@ __global__ __launch_bounds__(NW * 64) void k_conv_fwd(
   const bool live = *any_edges != 0;
   const unsigned long long dstep = DROP ? *dc.step : 0ull;
   const float sa = sgl::drop_scale(dc.p_att), so = sgl::drop_scale(dc.p_out);
+  if constexpr (DROP) {  // grid row p: dropout pass dc.pass + p, its own masks, saved state and output
+    to_pass(sv, d, size_t(gridDim.x) * RPW, blockIdx.y);
+    y += blockIdx.y * y_pass_stride;
+    dc.pass += blockIdx.y;
+  }
   if (nrows == 0 || !live) {
     // rows outside the live set: zero output (y's row U is the null
     // embedding the predictor's reductions read); a block without edges:
@@ -393,7 +422,7 @@ __global__ __launch_bounds__(NW * 64) void k_conv_fwd(
       L.AH[i * L.lda + D + j] = v;
     } else {
       v = cosf(p.te_b[j - D]);
-      if (i == 0 && blockIdx.x == 0 && sv.phi0 != nullptr) sv.phi0[j - D] = v;
+      if (i == 0 && blockIdx.x == 0 && blockIdx.y == 0 && sv.phi0 != nullptr) sv.phi0[j - D] = v;
     }
     L.HT[i * L.ldh + j] = v;
   }
@@ -406,6 +435,10 @@ __global__ __launch_bounds__(NW * 64) void k_conv_fwd(
   // in the edge loop.
   constexpr bool kPre = NW == 16;
   const bool staged = kPre && ts_rows > 0;
+  // the passes of one launch share X and S, whose encodings are the same in
+  // each: the first pass stores them (every pass of a 16-wave instance whose
+  // encodings do not fit in LDS, which reads its own back: the same values)
+  const bool te_store = !DROP || blockIdx.y == 0;
   if constexpr (BF) {
     const sgl::GemmJobBw jobs[1] = {{L.HT, L.ldh, bw.wq, bw.ld_q, p.b_q, L.Qs, L.ldr, D + T, D}};
     sgl::tile_gemm16_bw_jobs(jobs, kWaves);
@@ -427,8 +460,8 @@ __global__ __launch_bounds__(NW * 64) void k_conv_fwd(
             float sn, cs;
             te_sincos(te_arg(dtv, L.TW[t], L.TB[t]), sn, cs);
             if (staged) L.Ts[el * T + t] = cs;
-            X[row * C + D + d.F + t] = cs;
-            S[row * T + t] = sn;
+            if (te_store || !staged) X[row * C + D + d.F + t] = cs;
+            if (te_store) S[row * T + t] = sn;
           }
         }
         e += ntw;
@@ -578,7 +611,7 @@ __global__ __launch_bounds__(NW * 64) void k_conv_fwd(
 #pragma unroll
           for (int u = 0; u < kEC; ++u) {
             if (u < nv) {
-              fill_row<JM>(d, X, S, base + c0 + u, L.TW, L.TB, __shfl(my_dt, c0 + u - e0, 64), lane, x[u]);
+              fill_row<JM>(d, X, S, base + c0 + u, L.TW, L.TB, __shfl(my_dt, c0 + u - e0, 64), lane, te_store, x[u]);
             } else {
 #pragma unroll
               for (int j = 0; j < JM; ++j) x[u][j] = 0.f;
@@ -619,17 +652,19 @@ __global__ __launch_bounds__(NW * 64) void k_conv_fwd(
       // publish this slice's state for the merge (an empty slice has
       // m = -inf, l = 0, acc = 0 and drops out with weight e^-inf = 0)
 #pragma unroll
-      for (int h = 0; h < HM; ++h) {
-        if (h >= H) continue;
+      for (int h = 0; h < HL; ++h) {
+        const int hh = hg * HL + h;
+        if (hh >= H) continue;
+        const int ps = (i * NS + sl) * H + hh;
 #pragma unroll
         for (int j = 0; j < JM; ++j) {
           const int c = lane + 64 * j;
-          if (c < C) L.part[(wave * H + h) * C + c] = acc[h][j];
+          if (c < C) L.part[ps * C + c] = acc[h][j];
         }
         if (lane == 0) {
-          L.pml[(wave * H + h) * 3 + 0] = m[h];
-          L.pml[(wave * H + h) * 3 + 1] = l[h];
-          L.pml[(wave * H + h) * 3 + 2] = ls[h];
+          L.pml[ps * 3 + 0] = m[h];
+          L.pml[ps * 3 + 1] = l[h];
+          L.pml[ps * 3 + 2] = ls[h];
         }
       }
     }
@@ -644,10 +679,10 @@ __global__ __launch_bounds__(NW * 64) void k_conv_fwd(
       float v = 0.f, M = -INFINITY, Ls = 0.f, Lk = 0.f;
       if (s_cnt[i] > 0) {
 #pragma unroll
-        for (int s = 0; s < WPR; ++s) M = fmaxf(M, L.pml[((i * WPR + s) * H + h) * 3]);
+        for (int s = 0; s < NS; ++s) M = fmaxf(M, L.pml[((i * NS + s) * H + h) * 3]);
 #pragma unroll
-        for (int s = 0; s < WPR; ++s) {
-          const int w = i * WPR + s;
+        for (int s = 0; s < NS; ++s) {
+          const int w = i * NS + s;
           const float f = __expf(L.pml[(w * H + h) * 3] - M);
           Ls += L.pml[(w * H + h) * 3 + 1] * f;
           if (DROP) Lk += L.pml[(w * H + h) * 3 + 2] * f;
@@ -754,12 +789,12 @@ struct BwdLds {
   float *tep;                     // [waves][2][T]
   float *TB;                      // [T] time-encoding bias
   float *LG, *BK;                 // [D] LayerNorm weight, key bias (staged with the first loads)
-  float *part;                    // [NW][H*C]  a slice's G partial (slices only)
-  float *psig;                    // [NW][H]    a slice's sigma partial (slices only)
+  float *part;                    // [slices][H*C]  a slice's G partial (none with one slice a root)
+  float *psig;                    // [slices][H]    a slice's sigma partial
   float *scr;                     // [NW][4][64] four-row product partials (4-root tiles only)
 };
 
-__host__ __device__ inline BwdLds bwd_lds(const Dims &d, float *base, int nw, bool slices) {
+__host__ __device__ inline BwdLds bwd_lds(const Dims &d, float *base, int nw, int slices) {
   BwdLds L;
   L.ldr = sgl::lds_ld(d.D);
   L.ldq = sgl::lds_ld(d.H * d.C);
@@ -774,13 +809,13 @@ __host__ __device__ inline BwdLds bwd_lds(const Dims &d, float *base, int nw, bo
   L.LG = L.TB + d.T;
   L.BK = L.LG + d.D;
   L.part = L.BK + d.D;
-  L.psig = L.part + (slices ? nw * d.H * d.C : 0);
+  L.psig = L.part + slices * d.H * d.C;
   // 16-byte aligned for the product partials
-  L.scr = L.psig + (((slices ? nw * d.H : 0) + 3) & ~3);
+  L.scr = L.psig + ((slices * d.H + 3) & ~3);
   return L;
 }
 
-inline size_t bwd_lds_floats(const Dims &d, int nw, int rows, bool slices) {
+inline size_t bwd_lds_floats(const Dims &d, int nw, int rows, int slices) {
   float *base = reinterpret_cast<float *>(uintptr_t(4096));
   const BwdLds L = bwd_lds(d, base, nw, slices);
   return size_t(L.scr + (rows == 4 ? nw * 256 : 0) - base);
@@ -811,18 +846,19 @@ __global__ __launch_bounds__(NW * 64) void k_conv_bwd(
     const float *__restrict__ dt, ConvParams p,
     ConvSaved sv, const float *__restrict__ gy, long long *__restrict__ acc_src,
     long long *__restrict__ acc_dst, const float *__restrict__ w_s, const float *__restrict__ w_d,
-    float *__restrict__ g_src, float *__restrict__ g_dst, ConvGrads g, sgl::DropCfg dc, sgl_bf16_weights bw) {
+    float *__restrict__ g_src, float *__restrict__ g_dst, ConvGrads g, int64_t part_tiles, sgl::DropCfg dc,
+    sgl_bf16_weights bw) {
   constexpr int kWaves = NW, kBlock = NW * 64;
   constexpr int WPR = NW / RPW;
   constexpr int NS = WPR / HG;  // window slices per root (summed through LDS when > 1)
   constexpr int HL = HM / HG;   // heads per wave in the edge phase
   constexpr int EC = HG > 1 ? 2 : kEC;  // edges per round trip (fewer under the 1024-thread register cap)
   static_assert(RPW <= kRows && NW % RPW == 0 && NW <= kMaxWaves, "tile shape");
-  static_assert(WPR % HG == 0 && HM % HG == 0 && (HG == 1 || NS == 1), "head groups");
+  static_assert(WPR % HG == 0 && HM % HG == 0, "head groups");
   static_assert(!(BF && DROP), "the bf16 products run without dropout");
   extern __shared__ __align__(16) float lds[];
   const int D = d.D, T = d.T, H = d.H, C = d.C, dh = d.dh, K = d.k;
-  const BwdLds L = bwd_lds(d, lds, NW, NS > 1);
+  const BwdLds L = bwd_lds(d, lds, NW, NS > 1 ? RPW * NS : 0);
   __shared__ int s_cnt[kRows];
   __shared__ float s_sig[kRows][kMaxH];
 
@@ -833,6 +869,27 @@ __global__ __launch_bounds__(NW * 64) void k_conv_bwd(
   const bool live = *any_edges != 0;
   const unsigned long long dstep = DROP ? *dc.step : 0ull;
   const float sa = sgl::drop_scale(dc.p_att), so = sgl::drop_scale(dc.p_out);
+  if constexpr (DROP) {
+    // grid row p: dropout pass dc.pass + p, its own accumulator, saved state
+    // and gradients (the first pass's gradient comes through src_fc, the
+    // others' through dst_fc)
+    const int pass = blockIdx.y;
+    if (pass > 0) {
+      const size_t cap = size_t(gridDim.x) * RPW, rows = cap * pass;
+      to_pass(sv, d, cap, pass);
+      acc_src += pass * (cap + 1) * D;
+      g_src += pass * (cap + 1) * D;
+      w_s = w_d;
+      g.gz += rows * D;
+      g.gagg += rows * D;
+      g.gQ += rows * D;
+      g.G += rows * H * C;
+      g.sigma += rows * H;
+      g.ln_part += pass * part_tiles * 2 * D;
+      g.te_part += pass * part_tiles * 2 * T;
+      dc.pass += pass;
+    }
+  }
   // row U of the accumulators (the non-root negatives; row capacity when
   // every row is a root) belongs to the workgroup whose tile holds it, or
   // to the last one; the rows past U are never written by the predictor
@@ -1139,16 +1196,18 @@ __global__ __launch_bounds__(NW * 64) void k_conv_bwd(
           s_sig[i][hh] = sig[h];
         }
       }
-    } else {  // one head group (HL == HM): the slice's partials of every head
+    } else {  // the slice's partials of this wave's heads
 #pragma unroll
       for (int h = 0; h < HL; ++h) {
-        if (h >= H) continue;
+        const int hh = hg * HL + h;
+        if (hh >= H) continue;
+        const int ps = (i * NS + sl) * H + hh;
 #pragma unroll
         for (int j = 0; j < JM; ++j) {
           const int c = lane + 64 * j;
-          if (c < C) L.part[(wave * H + h) * C + c] = G[h][j];
+          if (c < C) L.part[ps * C + c] = G[h][j];
         }
-        if (lane == 0) L.psig[wave * H + h] = sig[h];
+        if (lane == 0) L.psig[ps] = sig[h];
       }
     }
   }
@@ -1170,7 +1229,7 @@ __global__ __launch_bounds__(NW * 64) void k_conv_bwd(
       const int i = idx / (H * C), hc = idx - i * (H * C), h = hc / C, c = hc - h * C;
       float v = 0.f;
 #pragma unroll
-      for (int s = 0; s < WPR; ++s) v += L.part[((i * WPR + s) * H + h) * C + c];
+      for (int s = 0; s < NS; ++s) v += L.part[((i * NS + s) * H + h) * C + c];
       L.GX[i * L.ldq + hc] = v;
       g.G[size_t(r0 + i) * H * C + hc] = v;
     }
@@ -1178,7 +1237,7 @@ __global__ __launch_bounds__(NW * 64) void k_conv_bwd(
       const int i = idx / H, h = idx - (idx / H) * H;
       float v = 0.f;
 #pragma unroll
-      for (int s = 0; s < WPR; ++s) v += L.psig[(i * WPR + s) * H + h];
+      for (int s = 0; s < NS; ++s) v += L.psig[(i * NS + s) * H + h];
       g.sigma[size_t(r0 + i) * H + h] = v;
       s_sig[i][h] = v;
     }
@@ -1279,6 +1338,8 @@ struct Instance {
   int waves;
   int rows;    // roots per workgroup
   int hg = 1;  // head groups per root in the edge phase
+  // window slices of the tile's roots together (0: one each, nothing to merge)
+  int slices() const { return waves / rows / hg > 1 ? waves / hg : 0; }
 };
 
 inline void instance_shape(const Dims &d, int &hm, int &jm) {
@@ -1392,7 +1453,7 @@ struct BwdPickDropWide {
 // the forward, the backward and sgl_conv_backward_tile_rows agree.
 bool fp32_four_fits(const Dims &d, int nw) {
   if (nw == 16) return true;
-  const bool slices = nw / kFp32Rows > 1;
+  const int slices = nw / kFp32Rows > 1 ? nw : 0;
   return sizeof(float) * fwd_lds_floats(d, nw, kFp32Rows, slices, 0) <= 160 * 1024 &&
          sizeof(float) * bwd_lds_floats(d, nw, kFp32Rows, slices) <= 160 * 1024;
 }
@@ -1516,21 +1577,24 @@ extern "C" int sgl_edge_rows(int32_t D, int32_t F, int32_t T, int32_t fanout, in
   return SGL_OK;
 }
 
-extern "C" int sgl_conv_forward(int32_t D, int32_t F, int32_t T, int32_t H, int32_t fanout, int64_t capacity,
+extern "C" int sgl_conv_forward_passes(int32_t D, int32_t F, int32_t T, int32_t H, int32_t fanout, int64_t capacity,
                                 const int32_t *num_roots, const int32_t *any_edges, const float *h_root,
                                 const int32_t *cnt, float *X, const float *dt, const float *w_q, const float *b_q,
                                 const float *w_k, const float *b_k, const float *w_v, const float *b_v,
                                 const float *w_out, const float *b_out, const float *ln_g, const float *ln_b,
                                 const float *te_w, const float *te_b, float *sv_Q, float *sv_qt, float *sv_xbar,
                                 float *sv_score, float *sv_ml, float *sv_agg, float *sv_z, float *sv_stats,
-                                float *sv_phi0, float *S, float *y, float p_att, float p_out, uint64_t seed,
-                                const uint64_t *rng_step, int32_t pass, float *sv_sdrop, const sgl_bf16_weights *bw,
-                                hipStream_t stream) {
+                                float *sv_phi0, float *S, float *y, int64_t y_pass_stride, float p_att, float p_out, uint64_t seed,
+                                const uint64_t *rng_step, int32_t pass, int32_t npass, float *sv_sdrop,
+                                const sgl_bf16_weights *bw, hipStream_t stream) {
   Dims d{D, F, T, H, D + F + T, H > 0 ? D / H : 0, fanout};
   if (int rc = check_dims(d)) return rc;
   sgl::DropCfg dc;
   bool drop;
   if (int rc = drop_cfg(p_att, p_out, seed, rng_step, pass, sv_sdrop, dc, drop)) return rc;
+  SGL_REQUIRE(npass == 1 || (drop && npass > 1 && npass <= kMaxPasses),
+              "conv_forward: %d passes (1, or up to %d with dropout)", npass, kMaxPasses);
+  SGL_REQUIRE(npass == 1 || y_pass_stride >= capacity * D, "conv_forward: the passes' outputs overlap");
   if (bw != nullptr)
     if (int rc = check_bf16_weights(d, *bw, drop)) return rc;
   SGL_REQUIRE(capacity >= 0 && capacity < INT_MAX && capacity % kRows == 0,
@@ -1545,7 +1609,7 @@ extern "C" int sgl_conv_forward(int32_t D, int32_t F, int32_t T, int32_t H, int3
                            : fp32_or_wide(d, pick_instance<FwdPick>(d), &pick_instance<FwdPickWide>);
   SGL_REQUIRE(inst.fn != nullptr, "conv_forward: no kernel instance for H=%d C=%d", H, d.C);
   // stage the tile's time encodings in LDS when they fit
-  const bool slices = inst.waves / inst.rows / inst.hg > 1;
+  const int slices = inst.slices();
   int ts_rows = fanout > 0 && T > 0 ? inst.rows * fanout : 0;
   if (sizeof(float) * fwd_lds_floats(d, inst.waves, inst.rows, slices, ts_rows) > 160 * 1024) ts_rows = 0;
   const size_t lds = sizeof(float) * fwd_lds_floats(d, inst.waves, inst.rows, slices, ts_rows);
@@ -1553,14 +1617,14 @@ extern "C" int sgl_conv_forward(int32_t D, int32_t F, int32_t T, int32_t H, int3
   SGL_CHECK_HIP(sgl::ensure_dynamic_lds(reinterpret_cast<const void *>(inst.fn), lds));
   ConvParams p{w_q, b_q, w_k, b_k, w_v, b_v, w_out, b_out, ln_g, ln_b, te_w, te_b};
   ConvSaved sv{sv_Q, sv_qt, sv_xbar, sv_score, sv_ml, sv_agg, sv_z, sv_stats, sv_phi0, sv_sdrop};
-  sgl::launch(inst.fn, dim3(unsigned(capacity / inst.rows)), dim3(unsigned(inst.waves * 64)), lds, stream, d,
-              num_roots, any_edges, h_root, cnt, X, dt, S, p, sv, y, ts_rows, dc,
+  sgl::launch(inst.fn, dim3(unsigned(capacity / inst.rows), unsigned(npass)), dim3(unsigned(inst.waves * 64)), lds, stream, d,
+              num_roots, any_edges, h_root, cnt, X, dt, S, p, sv, y, y_pass_stride, ts_rows, dc,
               bw != nullptr ? *bw : sgl_bf16_weights{});
   SGL_CHECK_LAUNCH();
   return SGL_OK;
 }
 
-extern "C" int sgl_conv_backward(int32_t D, int32_t F, int32_t T, int32_t H, int32_t fanout, int64_t capacity,
+extern "C" int sgl_conv_backward_passes(int32_t D, int32_t F, int32_t T, int32_t H, int32_t fanout, int64_t capacity,
                                  const int32_t *num_roots, const int32_t *any_edges, const int32_t *cnt,
                                  const float *X, const float *S, const float *dt, const float *w_q,
                                  const float *b_q, const float *w_k, const float *b_k, const float *w_v,
@@ -1571,14 +1635,16 @@ extern "C" int sgl_conv_backward(int32_t D, int32_t F, int32_t T, int32_t H, int
                                  int64_t *acc_src,
                                  int64_t *acc_dst, const float *w_s, const float *w_d, float *g_src, float *g_dst,
                                  float *gz, float *gagg, float *G, float *sigma, float *gQ, float *ln_part,
-                                 float *te_part, float p_att, float p_out, uint64_t seed, const uint64_t *rng_step,
-                                 int32_t pass, const float *sv_sdrop, const sgl_bf16_weights *bw,
-                                 hipStream_t stream) {
+                                 float *te_part, int64_t part_tiles, float p_att, float p_out, uint64_t seed,
+                                 const uint64_t *rng_step, int32_t pass, int32_t npass, const float *sv_sdrop,
+                                 const sgl_bf16_weights *bw, hipStream_t stream) {
   Dims d{D, F, T, H, D + F + T, H > 0 ? D / H : 0, fanout};
   if (int rc = check_dims(d)) return rc;
   sgl::DropCfg dc;
   bool drop;
   if (int rc = drop_cfg(p_att, p_out, seed, rng_step, pass, sv_sdrop, dc, drop)) return rc;
+  SGL_REQUIRE(npass == 1 || (drop && npass > 1 && npass <= kMaxPasses && gy == nullptr && acc_dst == nullptr && w_d),
+              "conv_backward: %d passes (1, or up to %d with dropout, from one accumulator each)", npass, kMaxPasses);
   if (bw != nullptr) {
     if (int rc = check_bf16_weights(d, *bw, drop)) return rc;
     SGL_REQUIRE(gy != nullptr || acc_dst != nullptr, "conv_backward: the bf16 products need both accumulators");
@@ -1600,7 +1666,8 @@ extern "C" int sgl_conv_backward(int32_t D, int32_t F, int32_t T, int32_t H, int
   // sgl_conv_backward_tile_rows (the dropout instances' rows are the fp32 ones)
   const int32_t tile_rows = sgl_conv_backward_tile_rows(D, F, T, H, bw != nullptr ? 1 : 0);
   SGL_REQUIRE(inst.rows == tile_rows, "conv_backward: %d roots per workgroup, %d per tile", inst.rows, tile_rows);
-  const size_t lds = sizeof(float) * bwd_lds_floats(d, inst.waves, inst.rows, inst.waves / inst.rows / inst.hg > 1);
+  SGL_REQUIRE(npass == 1 || part_tiles >= capacity / inst.rows, "conv_backward: the passes' partials overlap");
+  const size_t lds = sizeof(float) * bwd_lds_floats(d, inst.waves, inst.rows, inst.slices());
   SGL_REQUIRE(lds <= 160 * 1024, "conv_backward: %zu bytes of LDS needed (> 160 KiB)", lds);
   SGL_CHECK_HIP(sgl::ensure_dynamic_lds(reinterpret_cast<const void *>(inst.fn), lds));
   ConvParams p{w_q, b_q, w_k, b_k, w_v, b_v, w_out, b_out, ln_g, ln_b, nullptr, te_b};
@@ -1609,10 +1676,45 @@ extern "C" int sgl_conv_backward(int32_t D, int32_t F, int32_t T, int32_t H, int
                const_cast<float *>(sv_z),     const_cast<float *>(sv_stats), nullptr,
                const_cast<float *>(sv_sdrop)};
   ConvGrads g{gz, gagg, G, sigma, gQ, ln_part, te_part};
-  sgl::launch(inst.fn, dim3(unsigned(capacity / inst.rows)), dim3(unsigned(inst.waves * 64)), lds, stream, d,
+  sgl::launch(inst.fn, dim3(unsigned(capacity / inst.rows), unsigned(npass)), dim3(unsigned(inst.waves * 64)), lds, stream, d,
               num_roots, any_edges, cnt, X, S, dt, p, sv, gy,
               reinterpret_cast<long long *>(acc_src), reinterpret_cast<long long *>(acc_dst), w_s, w_d, g_src, g_dst,
-              g, dc, bw != nullptr ? *bw : sgl_bf16_weights{});
+              g, part_tiles, dc, bw != nullptr ? *bw : sgl_bf16_weights{});
   SGL_CHECK_LAUNCH();
   return SGL_OK;
+}
+
+extern "C" int sgl_conv_forward(int32_t D, int32_t F, int32_t T, int32_t H, int32_t fanout, int64_t capacity,
+                                const int32_t *num_roots, const int32_t *any_edges, const float *h_root,
+                                const int32_t *cnt, float *X, const float *dt, const float *w_q, const float *b_q,
+                                const float *w_k, const float *b_k, const float *w_v, const float *b_v,
+                                const float *w_out, const float *b_out, const float *ln_g, const float *ln_b,
+                                const float *te_w, const float *te_b, float *sv_Q, float *sv_qt, float *sv_xbar,
+                                float *sv_score, float *sv_ml, float *sv_agg, float *sv_z, float *sv_stats,
+                                float *sv_phi0, float *S, float *y, float p_att, float p_out, uint64_t seed,
+                                const uint64_t *rng_step, int32_t pass, float *sv_sdrop, const sgl_bf16_weights *bw,
+                                hipStream_t stream) {
+  return sgl_conv_forward_passes(D, F, T, H, fanout, capacity, num_roots, any_edges, h_root, cnt, X, dt, w_q, b_q, w_k,
+                                 b_k, w_v, b_v, w_out, b_out, ln_g, ln_b, te_w, te_b, sv_Q, sv_qt, sv_xbar, sv_score,
+                                 sv_ml, sv_agg, sv_z, sv_stats, sv_phi0, S, y, 0, p_att, p_out, seed, rng_step, pass, 1,
+                                 sv_sdrop, bw, stream);
+}
+
+extern "C" int sgl_conv_backward(int32_t D, int32_t F, int32_t T, int32_t H, int32_t fanout, int64_t capacity,
+                                 const int32_t *num_roots, const int32_t *any_edges, const int32_t *cnt,
+                                 const float *X, const float *S, const float *dt, const float *w_q, const float *b_q,
+                                 const float *w_k, const float *b_k, const float *w_v, const float *b_v,
+                                 const float *w_out, const float *b_out, const float *ln_g, const float *ln_b,
+                                 const float *te_b, const float *sv_Q, const float *sv_qt, const float *sv_xbar,
+                                 const float *sv_score, const float *sv_ml, const float *sv_agg, const float *sv_z,
+                                 const float *sv_stats, const float *gy, int64_t *acc_src, int64_t *acc_dst,
+                                 const float *w_s, const float *w_d, float *g_src, float *g_dst, float *gz,
+                                 float *gagg, float *G, float *sigma, float *gQ, float *ln_part, float *te_part,
+                                 float p_att, float p_out, uint64_t seed, const uint64_t *rng_step, int32_t pass,
+                                 const float *sv_sdrop, const sgl_bf16_weights *bw, hipStream_t stream) {
+  return sgl_conv_backward_passes(D, F, T, H, fanout, capacity, num_roots, any_edges, cnt, X, S, dt, w_q, b_q, w_k,
+                                  b_k, w_v, b_v, w_out, b_out, ln_g, ln_b, te_b, sv_Q, sv_qt, sv_xbar, sv_score, sv_ml,
+                                  sv_agg, sv_z, sv_stats, gy, acc_src, acc_dst, w_s, w_d, g_src, g_dst, gz, gagg, G,
+                                  sigma, gQ, ln_part, te_part, 0, p_att, p_out, seed, rng_step, pass, 1, sv_sdrop, bw,
+                                  stream);
 }

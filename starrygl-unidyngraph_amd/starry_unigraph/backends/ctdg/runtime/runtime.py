@@ -528,7 +528,8 @@ class CTDGOnlineRuntime:
                 if any(isinstance(a, int) and lo <= a < hi for a in args):
                     raise RuntimeError(f"launch plan: {name} in the front part reads the trained parameters")
         calls = front + back
-        return (_capi.pack_ops(calls), len(front), len(back), [c[0] for c in calls], calls)
+        # (a launch of several dropout passes goes by the single pass's name)
+        return (_capi.pack_ops(calls), len(front), len(back), [c[0].removesuffix("_passes") for c in calls], calls)
 
     def reset_plans(self) -> None:
         """Drop recorded plans (after buffers they reference change)."""

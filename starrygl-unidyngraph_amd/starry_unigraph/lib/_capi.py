@@ -17,7 +17,7 @@ import torch  # loads the HIP runtime first, so the library binds to the same on
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_NAME = "libstarrygl_mi355x.so"
 LIB_PATH = os.path.join(_HERE, LIB_NAME)
-ABI_VERSION = 22
+ABI_VERSION = 23
 
 SGL_DERR_NODE_RANGE = 1
 SGL_DERR_EID_RANGE = 2
@@ -35,6 +35,7 @@ _sz = ctypes.c_size_t
 
 # the attention's dropout arguments: p_att, p_out, seed, rng_step, pass, sv_sdrop
 _DROP = [ctypes.c_float, ctypes.c_float, ctypes.c_uint64, _vp, _i32, _vp]
+_DROPS = [*_DROP[:-1], _i32, _DROP[-1]]   # the several-pass calls: npass after pass
 
 # name -> (restype, argtypes); mirrors include/starrygl_mi355x.h
 SIGNATURES: dict[str, tuple] = {
@@ -73,6 +74,8 @@ SIGNATURES: dict[str, tuple] = {
     "sgl_edge_rows": (ctypes.c_int, [_i32] * 4 + [_i64] + [_vp] * 8),
     "sgl_conv_forward": (ctypes.c_int, [_i32] * 5 + [_i64] + [_vp] * 29 + _DROP + [_vp, _vp]),
     "sgl_conv_backward": (ctypes.c_int, [_i32] * 5 + [_i64] + [_vp] * 39 + _DROP + [_vp, _vp]),
+    "sgl_conv_forward_passes": (ctypes.c_int, [_i32] * 5 + [_i64] + [_vp] * 29 + [_i64] + _DROPS + [_vp, _vp]),
+    "sgl_conv_backward_passes": (ctypes.c_int, [_i32] * 5 + [_i64] + [_vp] * 39 + [_i64] + _DROPS + [_vp, _vp]),
     "sgl_dropout_masks": (ctypes.c_int, [_i64, _i32, _i32, _i32, ctypes.c_float, ctypes.c_float, ctypes.c_uint64,
                                          _vp, _i32, _vp, _vp, _vp]),
     "sgl_predictor": (ctypes.c_int, [_i64, _i32, _i64, _i32] + [_vp] * 20 + [_i64, _vp, _vp, _vp]),

@@ -504,12 +504,6 @@ class DeviceStep:
             "sgl_edge_rows", d.D, d.F, d.T, d.fanout, b.cap, P(b.num_roots), P(st.memory), P(efeat_all),
             P(hop.cnt), P(hop.nbr), P(hop.eid), P(b.X), self._s()), "sgl_edge_rows"))
 
-    def _at(self, t: torch.Tensor, p: int, rows: int | None = None) -> int:
-        """Pointer to pass p's block of a pass-stacked buffer (``rows``: the
-        block's element count when it is not the tensor's share)."""
-        n = t.numel() // self.buf.passes if rows is None else rows
-        return t.data_ptr() + p * n * t.element_size()
-
     def conv_forward(self, params: list[torch.Tensor], efeat_all: torch.Tensor, drop=None) -> torch.Tensor:
         """The attention forward over the edge rows of the last edge_rows()
         (it adds the rows' time encodings and their sines S). ``drop`` =
@@ -518,14 +512,18 @@ class DeviceStep:
         b, d, P = self.buf, self.dims, _capi.ptr
         te_w, te_b, w_q, b_q, w_k, b_k, w_v, b_v, w_out, b_out, ln_g, ln_b = params
         pa, po, seed = drop if drop is not None else (0.0, 0.0, 0)
-        for p in range(b.passes if drop is not None else 1):
-            a = lambda t: self._at(t, p)
+        args = (d.D, d.F, d.T, d.H, d.fanout, b.cap, P(b.num_roots), P(b.any_edges), P(b.new_mem), P(b.hop.cnt),
+                P(b.X), P(b.hop.dt), P(w_q), P(b_q), P(w_k), P(b_k), P(w_v), P(b_v), P(w_out), P(b_out), P(ln_g),
+                P(ln_b), P(te_w), P(te_b), P(b.Q), P(b.qt), P(b.xbar), P(b.score), P(b.ml), P(b.agg), P(b.z),
+                P(b.stats), P(b.phi0), P(b.S), P(b.y))
+        if drop is not None and b.passes > 1:   # every pass in one launch
             self._call("conv_forward", lambda: _capi.check(_capi.call(
-                "sgl_conv_forward", d.D, d.F, d.T, d.H, d.fanout, b.cap, P(b.num_roots), P(b.any_edges),
-                P(b.new_mem), P(b.hop.cnt), P(b.X), P(b.hop.dt), P(w_q), P(b_q), P(w_k), P(b_k), P(w_v), P(b_v),
-                P(w_out), P(b_out), P(ln_g), P(ln_b), P(te_w), P(te_b), a(b.Q), a(b.qt), a(b.xbar), a(b.score),
-                a(b.ml), a(b.agg), a(b.z), a(b.stats), P(b.phi0), P(b.S), self._at(b.y, p, b.y_rows * d.D),
-                pa, po, seed, P(b.rng_step), p, a(b.sdrop), self._bw(), self._s()), "sgl_conv_forward"))
+                "sgl_conv_forward_passes", *args, b.y_rows * d.D, pa, po, seed, P(b.rng_step), 0, b.passes,
+                P(b.sdrop), self._bw(), self._s()), "sgl_conv_forward_passes"))
+        else:
+            self._call("conv_forward", lambda: _capi.check(_capi.call(
+                "sgl_conv_forward", *args, pa, po, seed, P(b.rng_step), 0, P(b.sdrop), self._bw(), self._s()),
+                "sgl_conv_forward"))
         return b.y
 
     def predictor(self, n: int, train: bool, pred: list[torch.Tensor], out_grads: list[torch.Tensor] | None,
@@ -576,26 +574,31 @@ class DeviceStep:
         te_w, te_b, w_q, b_q, w_k, b_k, w_v, b_v, w_out, b_out, ln_g, ln_b = params
         hop = b.hop
         pa, po, seed = drop if drop is not None else (0.0, 0.0, 0)
-        passes = b.passes if drop is not None else 1
+        several = drop is not None and b.passes > 1   # every pass in one launch
+        acc_a = acc_b = g_a = g_b = w_a = w_b = None
         if gy is not None:
+            if several:
+                raise RuntimeError("conv_backward_kernel: the dropout passes take dL/dy from the predictor's rows")
             gy = gy.contiguous()
-        for p in range(passes):
-            if gy is not None:
-                acc_a = acc_b = g_a = g_b = w_a = w_b = None
-            elif passes == 1:
-                acc_a, acc_b, g_a, g_b = b.acc_src, b.acc_dst, b.g_src, b.g_dst
-                w_a, w_b = pred_w
-            else:
-                acc_a, g_a, w_a = b.acc_all[p], b.g_all[p], pred_w[0 if p == 0 else 1]
-                acc_b = g_b = w_b = None
-            a = lambda t: self._at(t, p)
+        elif several:
+            acc_a, g_a = b.acc_all, b.g_all
+            w_a, w_b = pred_w
+        else:
+            acc_a, acc_b, g_a, g_b = b.acc_src, b.acc_dst, b.g_src, b.g_dst
+            w_a, w_b = pred_w
+        args = (d.D, d.F, d.T, d.H, d.fanout, b.cap, P(b.num_roots), P(b.any_edges), P(hop.cnt), P(b.X), P(b.S),
+                P(hop.dt), P(w_q), P(b_q), P(w_k), P(b_k), P(w_v), P(b_v), P(w_out), P(b_out), P(ln_g), P(ln_b),
+                P(te_b), P(b.Q), P(b.qt), P(b.xbar), P(b.score), P(b.ml), P(b.agg), P(b.z), P(b.stats), P(gy),
+                P(acc_a), P(acc_b), P(w_a), P(w_b), P(g_a), P(g_b), P(b.gz), P(b.gagg), P(b.G), P(b.sigma), P(b.gQ),
+                P(b.ln_part), P(b.te_part))
+        if several:
             self._call("conv_backward", lambda: _capi.check(_capi.call(
-                "sgl_conv_backward", d.D, d.F, d.T, d.H, d.fanout, b.cap, P(b.num_roots), P(b.any_edges),
-                P(hop.cnt), P(b.X), P(b.S), P(hop.dt), P(w_q), P(b_q), P(w_k), P(b_k), P(w_v), P(b_v), P(w_out),
-                P(b_out), P(ln_g), P(ln_b), P(te_b), a(b.Q), a(b.qt), a(b.xbar), a(b.score), a(b.ml), a(b.agg),
-                a(b.z), a(b.stats), P(gy), P(acc_a), P(acc_b), P(w_a), P(w_b), P(g_a), P(g_b), a(b.gz), a(b.gagg),
-                a(b.G), a(b.sigma), a(b.gQ), a(b.ln_part), a(b.te_part), pa, po, seed, P(b.rng_step), p,
-                a(b.sdrop), self._bw(), self._s()), "sgl_conv_backward"))
+                "sgl_conv_backward_passes", *args, b.tiles, pa, po, seed, P(b.rng_step), 0, b.passes, P(b.sdrop),
+                self._bw(), self._s()), "sgl_conv_backward_passes"))
+        else:
+            self._call("conv_backward", lambda: _capi.check(_capi.call(
+                "sgl_conv_backward", *args, pa, po, seed, P(b.rng_step), 0, P(b.sdrop), self._bw(), self._s()),
+                "sgl_conv_backward"))
 
     def conv_backward(self, params: list[torch.Tensor], efeat_all: torch.Tensor, gy: torch.Tensor, drop=None):
         """The backward kernel plus the weight gradients as torch products (the
