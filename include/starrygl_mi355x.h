@@ -124,6 +124,17 @@ int sgl_recent_sample_packed(const int64_t *indptr, const int32_t *nbr_eid,
                              int32_t *out_eid, float *out_dt, int64_t *out_ts,
                              int32_t *err_flag, hipStream_t stream);
 
+/* That packed copy of a CSR (no reference counterpart: a layout of this
+ * build's sampler): nbr_eid [num_edges][2], ts32 [num_edges], fence
+ * [ceil(num_edges / 32)], and in flags (two int64, zero on entry) whether
+ * they may be used: flags[1] != 0: some timestamp does not fit in int32
+ * (use none of them); flags[0] != 0: some node's list is not sorted by time
+ * (pass no fence). */
+int sgl_recent_pack(int64_t num_nodes, int64_t num_edges, const int64_t *indptr,
+                    const int32_t *nbr, const int32_t *eid, const int64_t *ts,
+                    int32_t *nbr_eid, int32_t *ts32, int32_t *fence,
+                    int64_t *flags, hipStream_t stream);
+
 /* Padded -> the reference's concatenated layout (TemporalGraphBlock order:
  * root order, each window oldest->newest; output.h:4-30). out_ptr[Q+1] is the
  * exclusive scan of cnt, entry j of window i lands at out_ptr[i] + j. The

@@ -132,14 +132,21 @@ class RecentSampler:
         self.ids: torch.Tensor | None = None
         self.fence: torch.Tensor | None = None
         if narrow_ts and graph.num_edges > 0:
-            lo, hi = int(graph.ts.min().item()), int(graph.ts.max().item())
-            if -2 ** 31 <= lo and hi < 2 ** 31:
-                self.ts32 = graph.ts.to(torch.int32)
-                self.ids = torch.stack([graph.nbr, graph.eid], dim=1).contiguous()
-                # sorted lists: every decrease of ts is at a list boundary
-                down = torch.nonzero(graph.ts[1:] < graph.ts[:-1]).flatten() + 1
-                if down.numel() == 0 or bool(torch.isin(down, graph.indptr).all()):
-                    self.fence = self.ts32[::32].contiguous()
+            e, dev = graph.num_edges, self.dev
+            with torch.cuda.device(dev):
+                ids = torch.empty(e, 2, dtype=torch.int32, device=dev)
+                ts32 = torch.empty(e, dtype=torch.int32, device=dev)
+                fence = torch.empty((e + 31) // 32, dtype=torch.int32, device=dev)
+                flags = torch.zeros(2, dtype=torch.int64, device=dev)
+                P = _capi.ptr
+                _capi.check(_capi.lib().sgl_recent_pack(
+                    graph.num_nodes, e, P(graph.indptr), P(graph.nbr), P(graph.eid), P(graph.ts), P(ids), P(ts32),
+                    P(fence), P(flags), _capi.stream_of(dev)), "sgl_recent_pack")
+            unsorted, wide = flags.tolist()
+            if not wide:
+                self.ts32, self.ids = ts32, ids
+                if not unsorted:
+                    self.fence = fence
 
     @classmethod
     def for_graph(cls, graph: DeviceTCSR) -> "RecentSampler":
