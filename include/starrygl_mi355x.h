@@ -147,6 +147,26 @@ int sgl_recent_compact(int64_t num_queries, int32_t fanout, const int32_t *cnt,
                        int64_t *out_ptr, int32_t *out_nbr, int32_t *out_eid,
                        float *out_dt, int64_t *out_ts, void *workspace,
                        size_t workspace_bytes, hipStream_t stream);
+/* Its two halves, for a caller that sizes the outputs from the counts:
+ * sgl_recent_ptr writes ptr[0..Q] (the exclusive scan of cnt), and in meta
+ * (two int64, may be NULL) the total and *err_flag (0 without one), so that
+ * one host read gives both; sgl_recent_fill copies the entries to the places
+ * that ptr gives. */
+int sgl_recent_ptr(int64_t num_queries, const int32_t *cnt, int64_t *out_ptr,
+                   const int32_t *err_flag, int64_t *meta, void *workspace,
+                   size_t workspace_bytes, hipStream_t stream);
+int sgl_recent_fill(int64_t num_queries, int32_t fanout, const int64_t *ptr,
+                    const int32_t *pad_nbr, const int32_t *pad_eid,
+                    const float *pad_dt, const int64_t *pad_ts,
+                    int32_t *out_nbr, int32_t *out_eid, float *out_dt,
+                    int64_t *out_ts, hipStream_t stream);
+/* Per entry o of query q's window [ptr[q], ptr[q+1]) of a concatenated hop:
+ * index[o] = q, delta[o] = q_ts[q] - ts[o], place[o] = o - ptr[q] (each may be
+ * NULL; TemporalGraphBlock's src_index, delta_ts and sample_weight,
+ * output.h:4-30). No window is longer than fanout. */
+int sgl_block_index(int64_t num_queries, int32_t fanout, const int64_t *ptr,
+                    const int64_t *q_ts, const int64_t *ts, int64_t *index,
+                    int64_t *delta, float *place, hipStream_t stream);
 /* The same compaction without a workspace argument and without allocating:
  * its scratch (the per-tile count sums and offsets) is a static device array
  * of the library, 1 MiB per GPU, held until the process ends. No counterpart

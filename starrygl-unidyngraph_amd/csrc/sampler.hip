@@ -26,7 +26,10 @@
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kTile = 256;      // queries per compaction tile
+constexpr int kTile = 256;      // queries per workgroup of the compaction's copies
+constexpr int kSumPer = 4;      // queries per thread of its count sums
+constexpr int kSumTile = kBlock * kSumPer;
+constexpr int64_t kDirectTiles = 2048;  // above: the count tiles' offsets are scanned by a launch of their own
 constexpr int kScanBlock = 1024;
 constexpr int64_t kWaveModeMaxQueries = 1 << 15;  // below: one wavefront per query
 constexpr int64_t kFence = 32;  // CSR entries per fence (one 128-byte line of int32 times)
@@ -238,19 +241,78 @@ __global__ __launch_bounds__(kBlock) void k_recent_wave(
   }
 }
 
-__global__ __launch_bounds__(kTile) void k_tile_sums(int64_t nq, const int32_t *__restrict__ cnt,
-                                                     int64_t *__restrict__ tile_sum) {
-  const int64_t i = int64_t(blockIdx.x) * kTile + threadIdx.x;
-  const int64_t c = i < nq ? cnt[i] : 0;
-  __shared__ int64_t s_w[kTile / sgl::kWave];
+// ptr[0..nq]: the exclusive scan of the counts. A first launch sums each tile
+// of kSumTile counts; a second adds up the sums before its tile (or, with more
+// than kDirectTiles tiles, where that would read them too often, takes the
+// tile's offset from k_scan_tiles) and scans its own counts.
+__global__ __launch_bounds__(kBlock) void k_tile_sums(int64_t nq, const int32_t *__restrict__ cnt,
+                                                      int64_t *__restrict__ tile_sum) {
+  __shared__ int64_t s_w[kBlock / sgl::kWave];
+  const int64_t i0 = int64_t(blockIdx.x) * kSumTile + threadIdx.x;
+  int64_t c = 0;
+#pragma unroll
+  for (int u = 0; u < kSumPer; ++u) {
+    const int64_t i = i0 + u * kBlock;
+    if (i < nq) c += cnt[i];
+  }
   const int64_t s = sgl::wave_reduce_sum(c);
   if ((threadIdx.x & (sgl::kWave - 1)) == 0) s_w[threadIdx.x / sgl::kWave] = s;
   __syncthreads();
   if (threadIdx.x == 0) {
     int64_t tot = 0;
 #pragma unroll
-    for (int w = 0; w < kTile / sgl::kWave; ++w) tot += s_w[w];
+    for (int w = 0; w < kBlock / sgl::kWave; ++w) tot += s_w[w];
     tile_sum[blockIdx.x] = tot;
+  }
+}
+
+__global__ __launch_bounds__(kBlock) void k_write_ptr(int64_t nq, const int32_t *__restrict__ cnt,
+                                                      const int64_t *__restrict__ tile_sum,
+                                                      const int64_t *__restrict__ tile_off,
+                                                      int64_t *__restrict__ ptr, const int32_t *__restrict__ err,
+                                                      int64_t *__restrict__ meta) {
+  __shared__ int64_t s_w[kBlock / sgl::kWave];
+  __shared__ int64_t s_base;
+  int64_t base;
+  if (tile_off != nullptr) {
+    base = tile_off[blockIdx.x];
+  } else {
+    int64_t before = 0;
+    for (int64_t t = threadIdx.x; t < int64_t(blockIdx.x); t += kBlock) before += tile_sum[t];
+    const int64_t s = sgl::wave_reduce_sum(before);
+    if ((threadIdx.x & (sgl::kWave - 1)) == 0) s_w[threadIdx.x / sgl::kWave] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      int64_t tot = 0;
+#pragma unroll
+      for (int w = 0; w < kBlock / sgl::kWave; ++w) tot += s_w[w];
+      s_base = tot;
+    }
+    __syncthreads();
+    base = s_base;
+  }
+  // a thread's counts are consecutive: one scan of the threads' sums
+  const int64_t i0 = int64_t(blockIdx.x) * kSumTile + int64_t(threadIdx.x) * kSumPer;
+  int32_t c[kSumPer], sum = 0;
+#pragma unroll
+  for (int u = 0; u < kSumPer; ++u) {
+    c[u] = i0 + u < nq ? cnt[i0 + u] : 0;
+    sum += c[u];
+  }
+  __shared__ int32_t s_scan[kBlock / sgl::kWave];
+  int32_t total;
+  int64_t run = base + sgl::block_exclusive_scan<int32_t, kBlock>(sum, s_scan, total);
+#pragma unroll
+  for (int u = 0; u < kSumPer; ++u) {
+    if (i0 + u < nq) ptr[i0 + u] = run;
+    run += c[u];
+    if (i0 + u == nq - 1) {
+      ptr[nq] = run;
+      if (meta != nullptr) {
+        meta[0] = run;
+        meta[1] = err != nullptr ? *err : 0;
+      }
+    }
   }
 }
 
@@ -273,43 +335,73 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_tiles(
   }
 }
 
-__global__ __launch_bounds__(kTile) void k_compact_fill(
-    int64_t nq, int k, const int32_t *__restrict__ cnt,
-    const int64_t *__restrict__ tile_off, const int32_t *__restrict__ pnbr,
-    const int32_t *__restrict__ peid, const float *__restrict__ pdt,
-    const int64_t *__restrict__ pts, int64_t *__restrict__ out_ptr,
-    int32_t *__restrict__ out_nbr, int32_t *__restrict__ out_eid,
-    float *__restrict__ out_dt, int64_t *__restrict__ out_ts) {
+// Calls body(q, j, o) for every entry j of every query q < nq of this
+// workgroup's kTile queries, o its place in the concatenated output. Threads
+// walk the tile's padded slots (q, j < k), so that the padded rows are read and
+// the output written in order; the slot's query comes from adding, not from a
+// search of the tile's offsets. Bound by the bytes: 2 M entries (40 read and
+// written each) take 29 us. With the offsets scanned once and src_index /
+// delta_ts written by k_block_index (tensor operations before: a second scan,
+// repeat_interleave and two gathers a call), two hops of 20 from 8,000 queries
+// with their four getters take 140 us of kernels and 19 launches, before 244
+// us and 52: 380 -> 169 us with the host's part.
+template <class Body>
+__device__ __forceinline__ void for_tile_entries(int64_t nq, int k, const int64_t *__restrict__ ptr, Body body) {
   __shared__ int32_t s_off[kTile + 1];
-  __shared__ int32_t s_w[kTile / sgl::kWave];
   const int tid = threadIdx.x;
   const int64_t q0 = int64_t(blockIdx.x) * kTile;
-  const int64_t i = q0 + tid;
-  const int c = i < nq ? cnt[i] : 0;
-  int32_t total;
-  const int32_t off = sgl::block_exclusive_scan<int32_t, kTile>(c, s_w, total);
-  s_off[tid] = off;
-  if (tid == 0) s_off[kTile] = total;
-  const int64_t base = tile_off[blockIdx.x];
-  if (i < nq) out_ptr[i] = base + off;
-  if (i == nq - 1) out_ptr[nq] = base + off + c;
+  const int nt = int(min(int64_t(kTile), nq - q0));
+  const int64_t base = ptr[q0];
+  if (tid <= nt) s_off[tid] = int32_t(ptr[q0 + tid] - base);
+  if (tid == 0) s_off[nt] = int32_t(ptr[q0 + nt] - base);
   __syncthreads();
-  for (int j = tid; j < total; j += kTile) {
-    int lo = 0, hi = kTile;  // owner: the largest q with s_off[q] <= j
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if (s_off[mid] <= j) lo = mid; else hi = mid;
+  const int dq = kTile / k, dj = kTile - dq * k;
+  int q = tid / k, j = tid - q * k;
+  while (q < nt) {
+    if (j < s_off[q + 1] - s_off[q]) body(q0 + q, j, base + s_off[q] + j);
+    q += dq;
+    j += dj;
+    if (j >= k) {
+      j -= k;
+      ++q;
     }
-    const int64_t src = (q0 + lo) * k + (j - s_off[lo]);
-    const int64_t o = base + j;
+  }
+}
+
+__global__ __launch_bounds__(kTile) void k_compact_fill(
+    int64_t nq, int k, const int64_t *__restrict__ ptr, const int32_t *__restrict__ pnbr,
+    const int32_t *__restrict__ peid, const float *__restrict__ pdt, const int64_t *__restrict__ pts,
+    int32_t *__restrict__ out_nbr, int32_t *__restrict__ out_eid, float *__restrict__ out_dt,
+    int64_t *__restrict__ out_ts) {
+  for_tile_entries(nq, k, ptr, [&](int64_t q, int j, int64_t o) {
+    const int64_t src = q * k + j;
     out_nbr[o] = pnbr[src];
     out_eid[o] = peid[src];
     out_dt[o] = pdt[src];
     if (out_ts != nullptr) out_ts[o] = pts[src];
-  }
+  });
 }
 
-__global__ void k_write_zero_ptr(int64_t *out_ptr) { out_ptr[0] = 0; }
+// Per entry of a concatenated hop: its query, that query's time less the
+// entry's, and its place in the query's window.
+__global__ __launch_bounds__(kTile) void k_block_index(int64_t nq, int k, const int64_t *__restrict__ ptr,
+                                                       const int64_t *__restrict__ q_ts,
+                                                       const int64_t *__restrict__ ts, int64_t *__restrict__ index,
+                                                       int64_t *__restrict__ delta, float *__restrict__ place) {
+  for_tile_entries(nq, k, ptr, [&](int64_t q, int j, int64_t o) {
+    if (index != nullptr) index[o] = q;
+    if (delta != nullptr) delta[o] = q_ts[q] - ts[o];
+    if (place != nullptr) place[o] = float(j);
+  });
+}
+
+__global__ void k_write_zero_ptr(int64_t *out_ptr, const int32_t *err, int64_t *meta) {
+  out_ptr[0] = 0;
+  if (meta != nullptr) {
+    meta[0] = 0;
+    meta[1] = err != nullptr ? *err : 0;
+  }
+}
 
 }  // namespace
 
@@ -390,7 +482,7 @@ extern "C" size_t sgl_compact_workspace_bytes(int64_t num_queries) {
 namespace {
 
 // The checks and launches shared by both compaction entry points; tile_sum
-// and tile_off hold ceil(num_queries / kTile) entries each. Every entry is
+// and tile_off hold ceil(num_queries / kSumTile) entries each. Every entry is
 // written before it is read, so the scratch needs no clearing.
 int compact_checks(int64_t num_queries, int32_t fanout, const int32_t *cnt, const int32_t *pad_nbr,
                    const int32_t *pad_eid, const float *pad_dt, const int64_t *pad_ts, const int64_t *out_ptr,
@@ -407,23 +499,63 @@ int compact_checks(int64_t num_queries, int32_t fanout, const int32_t *cnt, cons
   return SGL_OK;
 }
 
+int ptr_run(int64_t num_queries, const int32_t *cnt, int64_t *out_ptr, int64_t *tile_sum, int64_t *tile_off,
+            const int32_t *err, int64_t *meta, hipStream_t stream) {
+  if (num_queries == 0) {
+    k_write_zero_ptr<<<1, 1, 0, stream>>>(out_ptr, err, meta);
+    SGL_CHECK_LAUNCH();
+    return SGL_OK;
+  }
+  const int64_t tiles = (num_queries + kSumTile - 1) / kSumTile;
+  if (tiles > 1) {
+    k_tile_sums<<<unsigned(tiles), kBlock, 0, stream>>>(num_queries, cnt, tile_sum);
+    SGL_CHECK_LAUNCH();
+  }
+  const bool scan = tiles > kDirectTiles;
+  if (scan) {
+    k_scan_tiles<<<1, kScanBlock, 0, stream>>>(tiles, tile_sum, tile_off);
+    SGL_CHECK_LAUNCH();
+  }
+  k_write_ptr<<<unsigned(tiles), kBlock, 0, stream>>>(num_queries, cnt, tile_sum, scan ? tile_off : nullptr, out_ptr,
+                                                      err, meta);
+  SGL_CHECK_LAUNCH();
+  return SGL_OK;
+}
+
+int fill_run(int64_t num_queries, int32_t fanout, const int64_t *ptr, const int32_t *pad_nbr, const int32_t *pad_eid,
+             const float *pad_dt, const int64_t *pad_ts, int32_t *out_nbr, int32_t *out_eid, float *out_dt,
+             int64_t *out_ts, hipStream_t stream) {
+  if (num_queries == 0 || fanout == 0) return SGL_OK;
+  const size_t tiles = (size_t(num_queries) + kTile - 1) / kTile;
+  k_compact_fill<<<unsigned(tiles), kTile, 0, stream>>>(num_queries, fanout, ptr, pad_nbr, pad_eid, pad_dt, pad_ts,
+                                                        out_nbr, out_eid, out_dt, out_ts);
+  SGL_CHECK_LAUNCH();
+  return SGL_OK;
+}
+
 int compact_run(int64_t num_queries, int32_t fanout, const int32_t *cnt, const int32_t *pad_nbr,
                 const int32_t *pad_eid, const float *pad_dt, const int64_t *pad_ts, int64_t *out_ptr,
                 int32_t *out_nbr, int32_t *out_eid, float *out_dt, int64_t *out_ts, int64_t *tile_sum,
                 int64_t *tile_off, hipStream_t stream) {
-  if (num_queries == 0) {
-    k_write_zero_ptr<<<1, 1, 0, stream>>>(out_ptr);
-    SGL_CHECK_LAUNCH();
-    return SGL_OK;
+  if (int rc = ptr_run(num_queries, cnt, out_ptr, tile_sum, tile_off, nullptr, nullptr, stream)) return rc;
+  return fill_run(num_queries, fanout, out_ptr, pad_nbr, pad_eid, pad_dt, pad_ts, out_nbr, out_eid, out_dt, out_ts,
+                  stream);
+}
+
+// The tile sums and offsets in a caller's workspace.
+int compact_scratch(int64_t num_queries, void *workspace, size_t workspace_bytes, int64_t *&tile_sum,
+                    int64_t *&tile_off) {
+  tile_sum = tile_off = nullptr;
+  if (num_queries == 0) return SGL_OK;
+  const size_t need = sgl_compact_workspace_bytes(num_queries);
+  if (workspace_bytes < need || workspace == nullptr) {
+    sgl::set_error("compact: workspace %zu bytes < required %zu", workspace_bytes, need);
+    return SGL_ERR_WORKSPACE;
   }
-  const size_t tiles = (size_t(num_queries) + kTile - 1) / kTile;
-  k_tile_sums<<<unsigned(tiles), kTile, 0, stream>>>(num_queries, cnt, tile_sum);
-  SGL_CHECK_LAUNCH();
-  k_scan_tiles<<<1, kScanBlock, 0, stream>>>(int64_t(tiles), tile_sum, tile_off);
-  SGL_CHECK_LAUNCH();
-  k_compact_fill<<<unsigned(tiles), kTile, 0, stream>>>(num_queries, fanout, cnt, tile_off, pad_nbr, pad_eid,
-                                                        pad_dt, pad_ts, out_ptr, out_nbr, out_eid, out_dt, out_ts);
-  SGL_CHECK_LAUNCH();
+  const size_t tiles = (size_t(num_queries) + kSumTile - 1) / kSumTile;
+  sgl::Carver c(workspace);
+  tile_sum = c.take<int64_t>(tiles);
+  tile_off = c.take<int64_t>(tiles);
   return SGL_OK;
 }
 
@@ -440,20 +572,44 @@ extern "C" int sgl_recent_compact(int64_t num_queries, int32_t fanout,
   int rc = compact_checks(num_queries, fanout, cnt, pad_nbr, pad_eid, pad_dt, pad_ts, out_ptr, out_nbr, out_eid,
                           out_dt, out_ts);
   if (rc != SGL_OK) return rc;
-  int64_t *tile_sum = nullptr, *tile_off = nullptr;
-  if (num_queries > 0) {
-    const size_t need = sgl_compact_workspace_bytes(num_queries);
-    if (workspace_bytes < need || workspace == nullptr) {
-      sgl::set_error("compact: workspace %zu bytes < required %zu", workspace_bytes, need);
-      return SGL_ERR_WORKSPACE;
-    }
-    const size_t tiles = (size_t(num_queries) + kTile - 1) / kTile;
-    sgl::Carver c(workspace);
-    tile_sum = c.take<int64_t>(tiles);
-    tile_off = c.take<int64_t>(tiles);
-  }
+  int64_t *tile_sum, *tile_off;
+  rc = compact_scratch(num_queries, workspace, workspace_bytes, tile_sum, tile_off);
+  if (rc != SGL_OK) return rc;
   return compact_run(num_queries, fanout, cnt, pad_nbr, pad_eid, pad_dt, pad_ts, out_ptr, out_nbr, out_eid, out_dt,
                      out_ts, tile_sum, tile_off, stream);
+}
+
+extern "C" int sgl_recent_ptr(int64_t num_queries, const int32_t *cnt, int64_t *out_ptr, const int32_t *err_flag,
+                              int64_t *meta, void *workspace, size_t workspace_bytes, hipStream_t stream) {
+  int rc = compact_checks(num_queries, 0, cnt, nullptr, nullptr, nullptr, nullptr, out_ptr, nullptr, nullptr, nullptr,
+                          nullptr);
+  if (rc != SGL_OK) return rc;
+  int64_t *tile_sum, *tile_off;
+  rc = compact_scratch(num_queries, workspace, workspace_bytes, tile_sum, tile_off);
+  if (rc != SGL_OK) return rc;
+  return ptr_run(num_queries, cnt, out_ptr, tile_sum, tile_off, err_flag, meta, stream);
+}
+
+extern "C" int sgl_recent_fill(int64_t num_queries, int32_t fanout, const int64_t *ptr, const int32_t *pad_nbr,
+                               const int32_t *pad_eid, const float *pad_dt, const int64_t *pad_ts, int32_t *out_nbr,
+                               int32_t *out_eid, float *out_dt, int64_t *out_ts, hipStream_t stream) {
+  int rc = compact_checks(num_queries, fanout, reinterpret_cast<const int32_t *>(ptr), pad_nbr, pad_eid, pad_dt,
+                          pad_ts, ptr, out_nbr, out_eid, out_dt, out_ts);
+  if (rc != SGL_OK) return rc;
+  return fill_run(num_queries, fanout, ptr, pad_nbr, pad_eid, pad_dt, pad_ts, out_nbr, out_eid, out_dt, out_ts,
+                  stream);
+}
+
+extern "C" int sgl_block_index(int64_t num_queries, int32_t fanout, const int64_t *ptr, const int64_t *q_ts,
+                               const int64_t *ts, int64_t *index, int64_t *delta, float *place, hipStream_t stream) {
+  SGL_REQUIRE(num_queries >= 0 && fanout >= 0 && fanout <= 4096, "block_index: bad sizes");
+  if (num_queries == 0 || fanout == 0) return SGL_OK;
+  SGL_REQUIRE(ptr != nullptr && (delta == nullptr || (q_ts && ts)), "block_index: NULL array");
+  const size_t tiles = (size_t(num_queries) + kTile - 1) / kTile;
+  SGL_REQUIRE(tiles < size_t(INT_MAX), "block_index: too many queries");
+  k_block_index<<<unsigned(tiles), kTile, 0, stream>>>(num_queries, fanout, ptr, q_ts, ts, index, delta, place);
+  SGL_CHECK_LAUNCH();
+  return SGL_OK;
 }
 
 // ---------------------------------------------------------------------------
@@ -462,7 +618,7 @@ extern "C" int sgl_recent_compact(int64_t num_queries, int32_t fanout,
 // process), so a caller that cannot allocate (HIP graph capture, a serving
 // loop) passes only its inputs and outputs. Calls that overlap on one GPU
 // share the array and race.
-static constexpr int64_t kNoAllocTiles = SGL_COMPACT_NOALLOC_MAX_QUERIES / kTile;
+static constexpr int64_t kNoAllocTiles = SGL_COMPACT_NOALLOC_MAX_QUERIES / kTile;  // (kSumTile-query tiles: a quarter of it in use)
 static __device__ __align__(256) int64_t scratch[2 * kNoAllocTiles];
 
 namespace {

@@ -49,6 +49,9 @@ SIGNATURES: dict[str, tuple] = {
     "sgl_recent_sample_packed": (ctypes.c_int, [_vp, _vp, _vp, _vp, _i64, _vp, ctypes.c_int, _vp, _i64, _vp, _vp,
                                                 _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "sgl_recent_pack": (ctypes.c_int, [_i64, _i64] + [_vp] * 9),
+    "sgl_recent_ptr": (ctypes.c_int, [_i64] + [_vp] * 5 + [_sz, _vp]),
+    "sgl_recent_fill": (ctypes.c_int, [_i64, _i32] + [_vp] * 10),
+    "sgl_block_index": (ctypes.c_int, [_i64, _i32] + [_vp] * 7),
     "sgl_compact_workspace_bytes": (_sz, [_i64]),
     "sgl_recent_compact": (ctypes.c_int, [_i64, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz,
                                           _vp]),

@@ -114,9 +114,7 @@ class TemporalGraphBlock:
     def src_index(self) -> torch.Tensor:
         if self._hop is None:
             return self._empty()
-        cnt = self._hop.ptr[1:] - self._hop.ptr[:-1]
-        q = torch.arange(cnt.numel(), device=cnt.device, dtype=torch.int64)
-        return torch.repeat_interleave(q, cnt, output_size=self._count())
+        return self._hop.index("query")
 
     def sample_nodes_ts(self) -> torch.Tensor:
         if self._hop is None:
@@ -126,14 +124,12 @@ class TemporalGraphBlock:
     def delta_ts(self) -> torch.Tensor:
         if self._hop is None:
             return self._empty()
-        return self._hop.q_ts[self.src_index()] - self._hop.ts[:self._count()]
+        return self._hop.index("delta")
 
     def sample_weight(self) -> torch.Tensor:
         if self._hop is None:
             return self._empty(torch.float32)
-        si = self.src_index()
-        pos = torch.arange(si.numel(), device=si.device, dtype=torch.int64) - self._hop.ptr[si]
-        return pos.float()
+        return self._hop.index("place")
 
     def row(self) -> torch.Tensor:
         return self._empty()
@@ -186,9 +182,10 @@ class ParallelSampler:
                 raise RuntimeError(f"{name} tensor must be one-dimensional")
         t0 = time.perf_counter()
         self._sampler.err.reset()
-        hops = self._sampler.sample_hops(nodes, root_ts.to(torch.int64), self.fanouts[:self.num_layers],
-                                         want_last_ts=True)
-        self._sampler.err.raise_if_set("neighbor_sample_from_nodes")
+        hops, bits = self._sampler._sample_hops(nodes, root_ts.to(torch.int64), self.fanouts[:self.num_layers],
+                                                want_last_ts=True)
+        if bits:
+            self._sampler.err.raise_if_set("neighbor_sample_from_nodes")
         self.ret = []
         total = 0
         for hop in hops:

@@ -65,10 +65,25 @@ class SampleHop:
     dt: torch.Tensor               # float32 [M]
     ts: torch.Tensor | None        # int64 [M]
     q_ts: torch.Tensor             # int64 [Q]
+    fanout: int                    # the longest a window can be
 
     @property
     def num_queries(self) -> int:
         return self.ptr.numel() - 1
+
+    def index(self, what: str) -> torch.Tensor:
+        """Per entry its query ("query", int64), that query's time less the
+        entry's ("delta", int64) or its place in the window ("place",
+        float32), by one kernel (sgl_block_index)."""
+        dev, P = self.ptr.device, _capi.ptr
+        out = torch.empty(self.count(), dtype=torch.float32 if what == "place" else torch.int64, device=dev)
+        if out.numel():
+            with torch.cuda.device(dev):
+                o = {what: P(out)}
+                _capi.check(_capi.lib().sgl_block_index(
+                    self.num_queries, self.fanout, P(self.ptr), P(self.q_ts), P(self.ts), o.get("query"),
+                    o.get("delta"), o.get("place"), _capi.stream_of(dev)), "sgl_block_index")
+        return out
 
     def count(self) -> int:
         return int(self.nbr.numel())
@@ -222,44 +237,48 @@ class RecentSampler:
     def compact(self, hop: PaddedHop) -> SampleHop:
         """Padded -> concatenated (the reference's TemporalGraphBlock layout).
         Synchronises once to size the output."""
-        dev = self.dev
+        return self._compact(hop)[0]
+
+    def _compact(self, hop: PaddedHop) -> tuple[SampleHop, int]:
+        """compact() and the sampler's error bits as they stood after the hop
+        (the one host read gives both)."""
+        dev, lib, P = self.dev, _capi.lib(), _capi.ptr
         nq = hop.num_queries
-        ptr = torch.empty(nq + 1, dtype=torch.int64, device=dev)
         with torch.cuda.device(dev):
-            if nq > 0:
-                torch.cumsum(hop.cnt, 0, out=ptr[1:])
-                ptr[0] = 0
-                m = int(ptr[-1].item())
-            else:
-                ptr.zero_()
-                m = 0
+            stream = _capi.stream_of(dev)
+            ptr = torch.empty(nq + 1, dtype=torch.int64, device=dev)
+            meta = torch.empty(2, dtype=torch.int64, device=dev)
+            ws_bytes = lib.sgl_compact_workspace_bytes(nq)
+            ws = _capi.workspace(ws_bytes, dev)
+            _capi.check(lib.sgl_recent_ptr(nq, P(hop.cnt), P(ptr), P(self.err.t), P(meta), P(ws), ws_bytes, stream),
+                        "sgl_recent_ptr")
+            m, bits = meta.tolist()
             # at least one element each, so no output pointer is NULL
             mm = max(m, 1)
             nbr = torch.empty(mm, dtype=torch.int32, device=dev)
             eid = torch.empty(mm, dtype=torch.int32, device=dev)
             dt = torch.empty(mm, dtype=torch.float32, device=dev)
             ts = torch.empty(mm, dtype=torch.int64, device=dev) if hop.ts is not None else None
-            pad = [hop.nbr, hop.eid, hop.dt, hop.ts]
-            if hop.nbr.numel() == 0:  # fanout 0: nothing to read, but keep pointers valid
-                one = torch.empty(1, dtype=torch.int64, device=dev)
-                pad = [one.view(torch.int32)[:1], one.view(torch.int32)[:1], one.view(torch.float32)[:1],
-                       one if hop.ts is not None else None]
-            ws_bytes = _capi.lib().sgl_compact_workspace_bytes(nq)
-            ws = _capi.workspace(ws_bytes, dev)
-            _capi.check(_capi.lib().sgl_recent_compact(
-                nq, hop.fanout, _capi.ptr(hop.cnt), _capi.ptr(pad[0]), _capi.ptr(pad[1]), _capi.ptr(pad[2]),
-                _capi.ptr(pad[3]), _capi.ptr(ptr), _capi.ptr(nbr), _capi.ptr(eid), _capi.ptr(dt), _capi.ptr(ts),
-                _capi.ptr(ws), ws_bytes, _capi.stream_of(dev)), "sgl_recent_compact")
-        return SampleHop(ptr, nbr[:m], eid[:m], dt[:m], None if ts is None else ts[:m], hop.q_ts)
+            if m > 0:
+                _capi.check(lib.sgl_recent_fill(nq, hop.fanout, P(ptr), P(hop.nbr), P(hop.eid), P(hop.dt), P(hop.ts),
+                                                P(nbr), P(eid), P(dt), P(ts), stream), "sgl_recent_fill")
+        return SampleHop(ptr, nbr[:m], eid[:m], dt[:m], None if ts is None else ts[:m], hop.q_ts, hop.fanout), bits
 
     def sample_hops(self, nodes: torch.Tensor, q_ts: torch.Tensor, fanouts: list[int],
                     want_last_ts: bool = False) -> list[SampleHop]:
         """The reference's concatenated multi-hop output (sampler.h:393-399):
         hop l+1 queries are hop l's concatenated (sample_nodes, sample_nodes_ts)."""
+        return self._sample_hops(nodes, q_ts, fanouts, want_last_ts)[0]
+
+    def _sample_hops(self, nodes: torch.Tensor, q_ts: torch.Tensor, fanouts: list[int],
+                     want_last_ts: bool = False) -> tuple[list[SampleHop], int]:
+        """sample_hops() and the error bits of every hop."""
         hops: list[SampleHop] = []
+        bits = 0
         for li, k in enumerate(fanouts):
             last = li == len(fanouts) - 1
-            hop = self.compact(self.sample(nodes, q_ts, k, want_ts=(not last) or want_last_ts))
+            hop, b = self._compact(self.sample(nodes, q_ts, k, want_ts=(not last) or want_last_ts))
+            bits |= b
             hops.append(hop)
             nodes, q_ts = hop.nbr, hop.ts
-        return hops
+        return hops, bits
