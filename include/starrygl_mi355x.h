@@ -723,6 +723,13 @@ int sgl_grad_adam(const sgl_grad_job *jobs, const int32_t *tile_job,
                   const int32_t *const *gates, const float *coef, float beta1,
                   float beta2, float eps, float weight_decay, uint16_t *shadow,
                   hipStream_t stream);
+/* The gradients of sgl_grad_adam's kind-0 jobs alone, written to grad (no
+ * update; kind-1 jobs and the jobs' segments and shadow offsets are not
+ * read). For a backward whose gradients go to the caller: the weight-gradient
+ * part of loss.backward() for TemporalTransformerConv (models.py:77-137). */
+int sgl_weight_grads(const sgl_grad_job *jobs, const int32_t *tile_job,
+                     int32_t num_tiles, const int32_t *num_roots, float *grad,
+                     hipStream_t stream);
 /* The bf16 copies of sgl_grad_adam's kind-0 jobs from the current
  * parameters (no update): after the parameters are set outside the fused
  * update (initialisation, a loaded checkpoint). No reference counterpart. */

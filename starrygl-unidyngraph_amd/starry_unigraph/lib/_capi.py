@@ -85,6 +85,7 @@ SIGNATURES: dict[str, tuple] = {
     "sgl_predictor": (ctypes.c_int, [_i64, _i32, _i64, _i32] + [_vp] * 20 + [_i64, _vp, _vp, _vp]),
     "sgl_link_metrics_work_doubles": (_i64, [_i32]),
     "sgl_link_metrics": (ctypes.c_int, [_i32, _i32, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _vp]),
+    "sgl_weight_grads": (ctypes.c_int, [_vp, _vp, _i32, _vp, _vp, _vp]),
     "sgl_adam_step": (ctypes.c_int, [_i64] + [_vp] * 6 + [ctypes.c_float] * 5 + [_vp]),
     "sgl_adam_advance": (ctypes.c_int, [_vp, _vp, _vp]),
     "sgl_time_next_launch": (ctypes.c_int, [_vp, _vp]),

@@ -20,6 +20,7 @@ the rest its back part (see the runtime's launch plans).
 from __future__ import annotations
 
 import ctypes
+import functools
 from dataclasses import dataclass
 
 import torch
@@ -358,6 +359,8 @@ class DeviceStep:
         # HIP events around each library call, or None
         self.timer: list | None = None
         self.timed: set[str] | None = None   # names to time (None = all)
+        # conv_backward's weight-gradient job tables over these buffers, by form
+        self._grads: tuple | None = None
         # bf16 weight copies for the attention / predictor products (Bf16Shadow), or None: fp32
         self.bf16: Bf16Shadow | None = None
 
@@ -601,41 +604,90 @@ class DeviceStep:
                 "sgl_conv_backward"))
 
     def conv_backward(self, params: list[torch.Tensor], efeat_all: torch.Tensor, gy: torch.Tensor, drop=None):
-        """The backward kernel plus the weight gradients as torch products (the
-        autograd path, one pass). Returns the 12 parameter gradients
-        (TimeEncode w, b; w_q, b_q, w_k, b_k, w_v, b_v, w_out, b_out, ln
-        weight, ln bias)."""
+        """The backward kernel and the weight gradients (the autograd path,
+        one pass; sgl_weight_grads, no host synchronisation). Returns the 12
+        parameter gradients (TimeEncode w, b; w_q, b_q, w_k, b_k, w_v, b_v,
+        w_out, b_out, ln weight, ln bias), views of one new buffer."""
         self.conv_backward_kernel(params, efeat_all, gy, drop=drop)
-        b, d = self.buf, self.dims
-        te_w, te_b, w_q, b_q, w_k, b_k, w_v, b_v, w_out, b_out, ln_g, ln_b = params
-        # weight gradients: per-root products reduced over the live root rows
-        # (the kernels leave the rows past them unwritten)
-        D, H, C, T = d.D, d.H, d.C, d.T
-        dh = D // H
-        c = int(b.num_roots.item())
-        gz, gagg, gQ, new_mem = b.gz[:c], b.gagg[:c], b.gQ[:c], b.new_mem[:c]
-        g_w_out = torch.cat([gz.t() @ b.agg[:c], gz.t() @ new_mem], dim=1)
-        g_b_out = gz.sum(0)
-        ga = gagg.reshape(c, H, dh).permute(1, 2, 0).contiguous()          # [H, dh, U]
-        g_w_v = torch.bmm(ga, b.xbar[:c].permute(1, 0, 2).contiguous()).reshape(D, C)
-        if drop is not None and drop[0] > 0:   # the kept weights sum to s_h, not 1
-            g_b_v = (gagg.reshape(c, H, dh) * b.sdrop[:c].unsqueeze(-1)).sum(0).reshape(D)
-        else:
-            g_b_v = gagg.sum(0)
-        qh = b.Q[:c].reshape(c, H, dh)
-        g_w_k = torch.bmm(qh.permute(1, 2, 0).contiguous(), b.G[:c].permute(1, 0, 2).contiguous()).reshape(D, C)
-        g_b_k = (qh * b.sigma[:c].unsqueeze(-1)).sum(0).reshape(D)
-        sq = gQ.sum(0)
-        phi0 = torch.cos(te_b)
-        g_w_q = torch.cat([gQ.t() @ new_mem, torch.outer(sq, phi0)], dim=1)
-        g_b_q = sq
-        nt = b.cap // self.bwd_tile_rows(self.bf16 is not None and drop is None)
-        g_ln_g = b.ln_part[:nt, 0].sum(0)
-        g_ln_b = b.ln_part[:nt, 1].sum(0)
-        te = b.te_part[:nt, :, :T].sum(0)
-        g_te_w = te[0].reshape(T, 1)
-        g_te_b = te[1]   # includes the query's cos(b) term (folded in by the kernel)
-        return [g_te_w, g_te_b, g_w_q, g_b_q, g_w_k, g_b_k, g_w_v, g_b_v, g_w_out, g_b_out, g_ln_g, g_ln_b]
+        att_drop = drop is not None and drop[0] > 0
+        key = (att_drop, self.bwd_tile_rows(self.bf16 is not None and drop is None))
+        if self._grads is None or self._grads[0] is not self.buf:
+            self._grads = (self.buf, {})
+        jobs, table, tiles, sizes = (self._grads[1].get(key) or self._weight_grad_jobs(params, *key))[:4]
+        flat = torch.empty(sum(sizes), dtype=torch.float32, device=self.dev)
+        P = _capi.ptr
+        self._call("weight_grads", lambda: _capi.check(_capi.call(
+            "sgl_weight_grads", jobs, table, tiles, P(self.buf.num_roots), P(flat), self._s()), "sgl_weight_grads"))
+        return [g.view(p.shape) for g, p in zip(flat.split_with_sizes(sizes), params)]
+
+    def _weight_grad_jobs(self, params: list[torch.Tensor], att_drop: bool, tile_rows: int) -> tuple:
+        """sgl_weight_grads' job and tile tables over this step's buffers (device
+        pointers, tile count) and the parameters' sizes; made once per form (the
+        gradients' addresses are the launch's)."""
+        sizes = [p.numel() for p in params]
+        offs = [sum(sizes[:i]) for i in range(len(sizes))]
+        jobs, tiles = [], []
+
+        def gemm(x1, s1, x2, s2, o, ldo, rows, cols, r_fixed=-1, **_):
+            tb = (cols + 15) // 16
+            tiles.append(torch.arange(((rows + 15) // 16) * tb, dtype=torch.int32) * 256 + len(jobs))
+            jobs.append(_capi.GradJob(x1=x1, x2=x2, s1=s1, s2=s2, off=o, ldo=ldo, rows=rows, cols=cols, kind=0,
+                                      r_fixed=r_fixed, tiles_b=tb, npass=1))
+
+        one = torch.ones(1, dtype=torch.float32, device=self.dev)
+        attention_grad_jobs(self.buf, self.dims, offs, one.data_ptr(), gemm, tile_rows, att_drop)
+        arr = (_capi.GradJob * len(jobs))(*jobs)
+        table = torch.cat(tiles)
+        raw = torch.cat([torch.frombuffer(bytearray(bytes(arr)), dtype=torch.int32), table]).to(self.dev)
+        at = raw.data_ptr()
+        made = self._grads[1][att_drop, tile_rows] = (at, at + ctypes.sizeof(arr), table.numel(), sizes, raw, one)
+        return made
+
+
+def attention_grad_jobs(b: "StepBuffers", d: "ConvDims", off, one: int, gemm, tile_rows: int, att_drop: bool,
+                        shf=lambda *a, **k: {}) -> None:
+    """The attention's weight gradients as reductions over the step's rows, in
+    the order of TemporalTransformerConv.kernel_params(): ``gemm(x1, s1, x2,
+    s2, off, ldo, rows, cols, r_fixed, ps1, ps2, shd)`` per job (pointers,
+    strides and the passes' strides in floats), ``off`` the 12 parameters'
+    element offsets, ``one`` a device 1.0, ``tile_rows`` the roots per tile of
+    the backward that ran, ``att_drop``: the attention's weights do not sum to
+    one (b_v's gradient takes the kept sums), ``shf`` a job's bf16-copy
+    fields."""
+    D, T, H, C = d.D, d.T, d.H, d.C
+    dh = D // H
+    c, ntiles = b.cap, b.tiles   # a pass's rows and its block of the per-tile partials
+    te_w, te_b, w_q, b_q, w_k, b_k, w_v, b_v, w_out, b_out, ln_g, ln_b = off
+
+    def at(t, k=0):
+        return t.data_ptr() + 4 * k
+
+    # rows of width w: pass stride c * w; the per-tile partials: ntiles * w
+    def conv(x1, s1, x2, s2, o, ldo, rows, cols, x1w=0, x2w=0, r_fixed=-1, shd=None):
+        gemm(x1, s1, x2, s2, o, ldo, rows, cols, r_fixed=r_fixed, ps1=x1w, ps2=x2w, shd=shd)
+
+    rt = -tile_rows   # per-tile partials: the tiles holding live rows (the others' are zero)
+    conv(at(b.te_part), 2 * T, one, 0, te_w, 1, T, 1, x1w=ntiles * 2 * T, r_fixed=rt)
+    conv(at(b.te_part, T), 2 * T, one, 0, te_b, 1, T, 1, x1w=ntiles * 2 * T, r_fixed=rt)
+    conv(at(b.gQ), D, at(b.new_mem), D, w_q, D + T, D, D, x1w=c * D, shd=shf("w_q"))
+    conv(at(b.gQ), D, at(b.phi0), 0, w_q + D, D + T, D, T, x1w=c * D, shd=shf("w_q", col0=D))
+    conv(at(b.gQ), D, one, 0, b_q, 1, D, 1, x1w=c * D)
+    for h in range(H):
+        conv(at(b.Q, h * dh), D, at(b.G, h * C), H * C, w_k + h * dh * C, C, dh, C, x1w=c * D, x2w=c * H * C,
+             shd=shf("w_k", h))
+        conv(at(b.Q, h * dh), D, at(b.sigma, h), H, b_k + h * dh, 1, dh, 1, x1w=c * D, x2w=c * H)
+        conv(at(b.gagg, h * dh), D, at(b.xbar, h * C), H * C, w_v + h * dh * C, C, dh, C, x1w=c * D, x2w=c * H * C,
+             shd=shf("w_v", h))
+    if att_drop:   # agg_h = W_v xbar'_h + s_h b_v[h]
+        for h in range(H):
+            conv(at(b.gagg, h * dh), D, at(b.sdrop, h), H, b_v + h * dh, 1, dh, 1, x1w=c * D, x2w=c * H)
+    else:
+        conv(at(b.gagg), D, one, 0, b_v, 1, D, 1, x1w=c * D)
+    conv(at(b.gz), D, at(b.agg), D, w_out, 2 * D, D, D, x1w=c * D, x2w=c * D, shd=shf("w_out"))
+    conv(at(b.gz), D, at(b.new_mem), D, w_out + D, 2 * D, D, D, x1w=c * D, shd=shf("w_out", col0=D))
+    conv(at(b.gz), D, one, 0, b_out, 1, D, 1, x1w=c * D)
+    conv(at(b.ln_part), 2 * D, one, 0, ln_g, 1, D, 1, x1w=ntiles * 2 * D, r_fixed=rt)
+    conv(at(b.ln_part, D), 2 * D, one, 0, ln_b, 1, D, 1, x1w=ntiles * 2 * D, r_fixed=rt)
 
 
 class StepParamUpdate:
@@ -693,9 +745,7 @@ class StepParamUpdate:
 
     def _jobs(self, conv_params, pred_params):
         b, d, opt = self.step.buf, self.step.dims, self.opt
-        D, T, H, C = d.D, d.T, d.H, d.C
-        dh = D // H
-        ntiles = b.tiles   # a pass's block of the per-tile partials
+        D = d.D
         tile_rows = self.step.bwd_tile_rows(self.shadow is not None)
         base = opt.flat.data_ptr()
 
@@ -724,8 +774,6 @@ class StepParamUpdate:
             jobs.append(job)
 
         P = self.passes
-        c = b.cap
-
         sh = self.shadow
 
         def shf(*a, **k):   # a job's bf16-copy fields (none without a shadow)
@@ -739,12 +787,6 @@ class StepParamUpdate:
                               **(shd or {})),
                 ((rows + 15) // 16) * tb)
 
-        # the attention's reductions run over every pass's rows (rows of
-        # width w: pass stride c * w; the per-tile partials: ntiles * w)
-        def conv(x1, s1, x2, s2, o, ldo, rows, cols, x1w=None, x2w=None, r_fixed=-1, shd=None):
-            gemm(x1, s1, x2, s2, o, ldo, rows, cols, r_fixed=r_fixed, npass=P,
-                 ps1=0 if x1w is None else x1w, ps2=0 if x2w is None else x2w, shd=shd)
-
         one = at(self.one)
         if self.kind == "projection":
             # the time projection's weight [D, 1] and bias [D] from the
@@ -755,30 +797,9 @@ class StepParamUpdate:
             gemm(at(b.proj_part, D), 2 * D, one, 0, off(pb), 1, D, 1, nt)
             self._pred_jobs(gemm, add, at, off, one, pred_params, 1)
             return self._check(jobs, tiles, conv_params, pred_params)
-        te_w, te_b, w_q, b_q, w_k, b_k, w_v, b_v, w_out, b_out, ln_g, ln_b = conv_params
-        # per-tile partials: the tiles holding live rows (the others' are zero)
-        rt = -tile_rows
-        conv(at(b.te_part), 2 * T, one, 0, off(te_w), 1, T, 1, x1w=ntiles * 2 * T, r_fixed=rt)
-        conv(at(b.te_part, T), 2 * T, one, 0, off(te_b), 1, T, 1, x1w=ntiles * 2 * T, r_fixed=rt)
-        conv(at(b.gQ), D, at(b.new_mem), D, off(w_q), D + T, D, D, x1w=c * D, shd=shf("w_q"))
-        conv(at(b.gQ), D, at(b.phi0), 0, off(w_q) + D, D + T, D, T, x1w=c * D, shd=shf("w_q", col0=D))
-        conv(at(b.gQ), D, one, 0, off(b_q), 1, D, 1, x1w=c * D)
-        for h in range(H):
-            conv(at(b.Q, h * dh), D, at(b.G, h * C), H * C, off(w_k) + h * dh * C, C, dh, C, x1w=c * D,
-                 x2w=c * H * C, shd=shf("w_k", h))
-            conv(at(b.Q, h * dh), D, at(b.sigma, h), H, off(b_k) + h * dh, 1, dh, 1, x1w=c * D, x2w=c * H)
-            conv(at(b.gagg, h * dh), D, at(b.xbar, h * C), H * C, off(w_v) + h * dh * C, C, dh, C, x1w=c * D,
-                 x2w=c * H * C, shd=shf("w_v", h))
-        if P > 1:   # attention dropout: agg_h = W_v xbar'_h + s_h b_v[h]
-            for h in range(H):
-                conv(at(b.gagg, h * dh), D, at(b.sdrop, h), H, off(b_v) + h * dh, 1, dh, 1, x1w=c * D, x2w=c * H)
-        else:
-            conv(at(b.gagg), D, one, 0, off(b_v), 1, D, 1, x1w=c * D)
-        conv(at(b.gz), D, at(b.agg), D, off(w_out), 2 * D, D, D, x1w=c * D, x2w=c * D, shd=shf("w_out"))
-        conv(at(b.gz), D, at(b.new_mem), D, off(w_out) + D, 2 * D, D, D, x1w=c * D, shd=shf("w_out", col0=D))
-        conv(at(b.gz), D, one, 0, off(b_out), 1, D, 1, x1w=c * D)
-        conv(at(b.ln_part), 2 * D, one, 0, off(ln_g), 1, D, 1, x1w=ntiles * 2 * D, r_fixed=rt)
-        conv(at(b.ln_part, D), 2 * D, one, 0, off(ln_b), 1, D, 1, x1w=ntiles * 2 * D, r_fixed=rt)
+        # the attention's reductions run over every pass's rows
+        attention_grad_jobs(b, d, [off(p) for p in conv_params], one, functools.partial(gemm, npass=P), tile_rows, P > 1,
+                            shf)
         # edge predictor: src_fc / dst_fc as reductions over roots 0..U (row U
         # of g_dst holds the non-root negatives; y's row U is zero); out_fc's
         # gradients come from sgl_predictor (Adam only). With dropout dst_fc

@@ -1,0 +1,64 @@
+"""The attention backward's weight gradients (sgl_weight_grads: reductions over
+the step's rows by one launch) against the same products in float64 of the rows
+the backward kernel left, at root counts around the reduction's groups of 4 and
+tiles of 16, odd widths, one to four heads, the attention dropout's kept sums,
+and a block without roots. A sum of U float32 products in any order is within
+U * 2^-24 of the sum of their magnitudes."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("D,F,T,H,U,pa", [(32, 6, 16, 2, 1, 0.0), (30, 5, 7, 3, 15, 0.0), (44, 1, 20, 4, 17, 0.3),
+                                          (100, 172, 100, 2, 130, 0.0), (33, 0, 9, 1, 64, 0.2), (32, 6, 16, 2, 0, 0.0)])
+def test_weight_grads_match_float64_products(gpu, D, F, T, H, U, pa):
+    from starry_unigraph.native.step import ConvDims, DeviceStep, NodeState
+    k, N, E = 6, 80, 200
+    g = torch.Generator().manual_seed(D + U)
+    r = lambda *s: torch.randn(*s, generator=g).to(gpu)
+    state = NodeState(N, D, 1, F, gpu)
+    state.memory.copy_(r(N, D))
+    step = DeviceStep(state, ConvDims(D, F, T, H, k), max(U, 1))
+    b = step.buf
+    b.num_roots.fill_(U)
+    b.any_edges.fill_(1)
+    b.rng_step.fill_(3)
+    b.new_mem.copy_(r(b.cap, D))
+    b.hop.cnt.copy_(torch.randint(0, k + 1, (b.cap,), generator=g, dtype=torch.int32))
+    b.hop.nbr.copy_(torch.randint(0, N, (b.cap * k,), generator=g, dtype=torch.int32))
+    b.hop.eid.copy_(torch.randint(0, E, (b.cap * k,), generator=g, dtype=torch.int32))
+    b.hop.dt.copy_(torch.rand(b.cap * k, generator=g) * 1e3)
+    C, dh = D + F + T, D // H
+    params = [0.1 * r(T, 1), r(T), r(D, D + T) / D ** 0.5, r(D), r(D, C) / C ** 0.5, r(D), r(D, C) / C ** 0.5, r(D),
+              r(D, 2 * D) / D ** 0.5, r(D), r(D), r(D)]
+    drop = (pa, 0.0, 5) if pa > 0 else None
+    feat = r(E, max(F, 1))[:, :F].contiguous()
+    step.edge_rows(feat)
+    step.conv_forward(params, feat, drop=drop)
+    got = step.conv_backward(params, feat, r(b.y_rows, D), drop=drop)
+    again = step.conv_backward(params, feat, torch.zeros(b.y_rows, D, device=gpu), drop=drop)
+    assert all(x.data_ptr() != y.data_ptr() for x, y in zip(got, again))   # every call its own gradients
+    got2 = step.conv_backward(params, feat, r(b.y_rows, D), drop=drop)
+    nt = b.cap // step.bwd_tile_rows()
+    d = lambda t: t[:U].double()
+    one = torch.ones(U, 1, dtype=torch.float64, device=gpu)
+    heads = lambda t, h: d(t)[:, h * dh:(h + 1) * dh]
+    pairs = [None, None, (d(b.gQ), torch.cat([d(b.new_mem), b.phi0.double().expand(U, T)], 1)), (d(b.gQ), one),
+             [(heads(b.Q, h), d(b.G)[:, h]) for h in range(H)], [(heads(b.Q, h), d(b.sigma)[:, h:h + 1]) for h in range(H)],
+             [(heads(b.gagg, h), d(b.xbar)[:, h]) for h in range(H)],
+             [(heads(b.gagg, h), d(b.sdrop)[:, h:h + 1] if pa > 0 else one) for h in range(H)],
+             (d(b.gz), torch.cat([d(b.agg), d(b.new_mem)], 1)), (d(b.gz), one), None, None]
+    for i, (x, p) in enumerate(zip(got2, params)):
+        assert x.shape == p.shape
+        if pairs[i] is None:   # per-tile partials
+            part = {0: b.te_part[:nt, 0], 1: b.te_part[:nt, 1], 10: b.ln_part[:nt, 0], 11: b.ln_part[:nt, 1]}[i].double()
+            want, size = part.sum(0), part.abs().sum(0)
+        else:
+            ps = pairs[i] if isinstance(pairs[i], list) else [pairs[i]]
+            want = torch.cat([u.T @ v for u, v in ps])
+            size = torch.cat([u.abs().T @ v.abs() for u, v in ps])
+        want, size = want.reshape(p.shape), size.reshape(p.shape)
+        assert bool(((x.double() - want).abs() <= (U + 8) * 2.0 ** -24 * size).all()), i
+    if U == 0:
+        assert all(bool((x == 0).all()) for x in got2)
