@@ -273,6 +273,39 @@ int sgl_memory_update(int32_t D, int32_t K, int32_t F, int64_t capacity,
                       const uint64_t *win_src, const uint64_t *win_dst,
                       const int32_t *cnt_src, const int32_t *cnt_dst,
                       float *new_mem, hipStream_t stream);
+/* The same update and sgl_memory_commit (below) for small batches, together
+ * two launches that spread the roots' products over the GPU, through a
+ * workspace of sgl_memory_update_workspace_bytes(D, K, F, capacity) bytes; that
+ * query returns 0 where the two entry points are the better way (or the shape
+ * is not supported). Arguments: sgl_memory_update's, then the commit's that it
+ * does not share; the same bits as the two calls. */
+size_t sgl_memory_update_workspace_bytes(int32_t D, int32_t K, int32_t F, int64_t capacity);
+int sgl_memory_update_commit(int32_t D, int32_t K, int32_t F, int64_t capacity,
+                             const int32_t *num_roots, const int64_t *roots,
+                             float *memory, float *mailbox, float *mailbox_ts,
+                             int32_t *next_mail_pos, const float *w_ih,
+                             const float *w_hh, const float *b_ih, const float *b_hh,
+                             const float *wc_ih, const float *wc_hh,
+                             const float *bc_ih, const float *bc_hh,
+                             const int64_t *src, const int64_t *dst,
+                             const float *efeat, const float *ts,
+                             const int64_t *batch_start,
+                             const uint64_t *win_src, const uint64_t *win_dst,
+                             const int32_t *cnt_src, const int32_t *cnt_dst,
+                             float *new_mem, float *memory_ts, const float *ts_max,
+                             uint32_t *node_bits, const int32_t *sample_cnt,
+                             int32_t *any_edges, float *root_dt, void *workspace,
+                             size_t workspace_bytes, hipStream_t stream);
+/* CTDGMemoryUpdater.forward on rows given as they are (models.py:244-254):
+ * new_mem[r] from mailbox[r] [K][2D+F] and memory[r] [D] for r < rows, with
+ * sgl_memory_update_workspace_bytes of workspace for that many rows. Nothing
+ * else is written. */
+int sgl_memory_rows(int32_t D, int32_t K, int32_t F, int64_t rows,
+                    const float *memory, const float *mailbox, const float *w_ih,
+                    const float *w_hh, const float *b_ih, const float *b_hh,
+                    const float *wc_ih, const float *wc_hh, const float *bc_ih,
+                    const float *bc_hh, float *new_mem, void *workspace,
+                    size_t workspace_bytes, hipStream_t stream);
 /* The same update with the GRU's four weight matrices in bf16 (raw 16-bit
  * patterns, the same layouts): its GEMMs run on bf16 MFMA with fp32
  * accumulation, the mailbox rows, hidden state and memory rounded to bf16 as

@@ -88,7 +88,7 @@ __device__ __forceinline__ void gate_wait(const uint32_t *word, uint32_t value, 
 template <typename F, typename... Args>
 inline void launch(F kernel, dim3 grid, dim3 block, size_t lds, hipStream_t stream, Args... args) {
   LaunchTimer &t = pending_timer();
-  if (t.start != nullptr) {
+  if (t.start != nullptr || t.stop != nullptr) {
     const LaunchTimer u = t;
     t = LaunchTimer{nullptr, nullptr};
     hipExtLaunchKernelGGL(kernel, grid, block, uint32_t(lds), stream, u.start, u.stop, 0u, args...);

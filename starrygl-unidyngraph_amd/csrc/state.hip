@@ -16,6 +16,7 @@
 #include <climits>
 
 #include "common.h"
+#include "gru.h"
 #include "metrics.h"
 #include "mfma.h"
 
@@ -639,17 +640,6 @@ __device__ __forceinline__ float gate_tanh(float x) {
   return 1.f - 2.f * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(2.88539008f * x));
 }
 
-// GRU gate combination (PyTorch order r, z, n):
-//   r = s(gi_r + gh_r), z = s(gi_z + gh_z), n = tanh(gi_n + r * gh_n),
-//   h' = (1 - z) * n + z * h
-__device__ __forceinline__ float gru_combine(float gir, float giz, float gin, float ghr, float ghz,
-                                             float ghn, float h) {
-  const float r = 1.f / (1.f + expf(-(gir + ghr)));
-  const float z = 1.f / (1.f + expf(-(giz + ghz)));
-  const float n = tanhf(gin + r * ghn);
-  return (1.f - z) * n + z * h;
-}
-
 constexpr int kGruBlock = 1024;
 constexpr int kGruWaves = kGruBlock / sgl::kWave;
 constexpr int kMaxMsgSlots = 8;  // S = 2D + F <= 512
@@ -813,7 +803,7 @@ __global__ __launch_bounds__(kGruBlock) void k_gru_mailbox(
         } else {  // W_hh h0 = 0
           ghr = b_hh[j]; ghz = b_hh[D + j]; ghn = b_hh[2 * D + j];
         }
-        const float hv = gru_combine(g1[j], g1[D + j], g1[2 * D + j], ghr, ghz, ghn, hs[i * ldh + j]);
+        const float hv = sgl::gru_combine(g1[j], g1[D + j], g1[2 * D + j], ghr, ghz, ghn, hs[i * ldh + j]);
         hs[i * ldh + j] = hv;
         if constexpr (kBf) hb[i * lbh + j] = to_bf(hv);
       }
@@ -830,7 +820,7 @@ __global__ __launch_bounds__(kGruBlock) void k_gru_mailbox(
       const float *g1 = gi + i * ldg;
       const float *g2 = gh + i * ldg;
       new_mem[size_t(r0 + i) * D + j] =
-          gru_combine(g1[j], g1[D + j], g1[2 * D + j], g2[j], g2[D + j], g2[2 * D + j], ms[i * ldh + j]);
+          sgl::gru_combine(g1[j], g1[D + j], g1[2 * D + j], g2[j], g2[D + j], g2[2 * D + j], ms[i * ldh + j]);
     }
 
     // Mailbox write: the src-role message goes to slot p = next_mail_pos[u],

@@ -164,6 +164,17 @@ class CTDGMemoryUpdater(nn.Module):
         Fd = S - 2 * D
         mail = mailbox_history.to(dev, torch.float32).contiguous()
         mem = current_memory.to(dev, torch.float32).contiguous()
+        P = _capi.ptr
+        if self.gemm_dtype == "fp32":
+            n = int(_capi.lib().sgl_memory_update_workspace_bytes(D, K, Fd, M))
+            if n > 0:
+                w, ws = self.kernel_weights(), _capi.workspace(n, dev)
+                out = torch.empty(M, D, dtype=torch.float32, device=dev)
+                _capi.check(_capi.lib().sgl_memory_rows(
+                    D, K, Fd, M, P(mem), P(mail), P(w["w_ih"]), P(w["w_hh"]), P(w["b_ih"]), P(w["b_hh"]), P(w["wc_ih"]),
+                    P(w["wc_hh"]), P(w["bc_ih"]), P(w["bc_hh"]), P(out), P(ws), n, _capi.stream_of(dev)),
+                    "sgl_memory_rows")
+                return out
         cap = (M + 15) // 16 * 16
         roots = torch.arange(M, dtype=torch.int64, device=dev)
         n = torch.tensor([M], dtype=torch.int32, device=dev)
@@ -171,7 +182,6 @@ class CTDGMemoryUpdater(nn.Module):
         zeros_k = torch.zeros(cap, dtype=torch.int64, device=dev)
         out = torch.empty(cap, D, dtype=torch.float32, device=dev)
         w = self.kernel_weights()
-        P = _capi.ptr
         dummy_i64 = torch.zeros(1, dtype=torch.int64, device=dev)
         dummy_f = torch.zeros(max(Fd, 1), dtype=torch.float32, device=dev)
         mts = torch.zeros(M, K, dtype=torch.float32, device=dev)

@@ -528,8 +528,9 @@ class CTDGOnlineRuntime:
                 if any(isinstance(a, int) and lo <= a < hi for a in args):
                     raise RuntimeError(f"launch plan: {name} in the front part reads the trained parameters")
         calls = front + back
-        # (a launch of several dropout passes goes by the single pass's name)
-        return (_capi.pack_ops(calls), len(front), len(back), [c[0].removesuffix("_passes") for c in calls], calls)
+        # (another form of an entry point goes by the entry point's name)
+        names = [{"sgl_memory_update_commit": "sgl_memory_update"}.get(c[0], c[0].removesuffix("_passes")) for c in calls]
+        return (_capi.pack_ops(calls), len(front), len(back), names, calls)
 
     def reset_plans(self) -> None:
         """Drop recorded plans (after buffers they reference change)."""
@@ -539,8 +540,8 @@ class CTDGOnlineRuntime:
 
     def _front_body(self, step: DeviceStep, split: str, n: int, src, dst, neg, ts, ef, cursor,
                     prev_metrics: int = 0) -> None:
-        """Batch preparation, sampling and the GRU memory update of one step.
-        With ``cursor`` (device int64 [1]) the event and negative arrays are
+        """Batch preparation, sampling, the GRU memory update and its commit of
+        one step. With ``cursor`` (device int64 [1]) the event and negative arrays are
         the whole stream and the batch starts at the cursor (which the step
         advances). ``prev_metrics`` > 0: first the metrics of the previous
         step on these buffers (that many events), whose back part the
@@ -551,19 +552,18 @@ class CTDGOnlineRuntime:
         else:
             step.prepare(src, dst, neg, ts, n=n, cursor=cursor)
         step.sample(self.sampler.device_sampler("test" if split == "predict" else split))
+        # the memory update, then its commit (which also sets the step's "block
+        # has edges" gate)
         if self._gru is not None:
-            step.update_memory(self._gru, src, dst, ef, ts, from_cursor=cursor is not None)
+            step.update_and_commit(self._gru, src, dst, ef, ts, from_cursor=cursor is not None)
+        else:   # runtime.py:283-285: the conv reads the memory as it is
+            step.gather_memory()
 
     def _commit_body(self, step: DeviceStep, train: bool) -> None:
-        """The memory commit (which also sets the step's "block has edges"
-        gate), the sampled edges' rows from the committed memory (no trained
+        """After the memory commit: the sampled edges' rows (no trained
         parameter is read, so this may run beside the previous step's update)
         and, in training, the Adam step-count advance and bias corrections
         that the step's fused update reads."""
-        if self._gru is not None:
-            step.commit()
-        else:   # runtime.py:283-285: the conv reads the memory as it is
-            step.gather_memory()
         if not self._proj:
             step.edge_rows(self._dev["edge_feat"])
         if train:

@@ -64,6 +64,9 @@ SIGNATURES: dict[str, tuple] = {
     "sgl_memory_update_lds_bytes": (_sz, [_i32, _i32]),
     "sgl_memory_update_bf16_tile_rows": (_i32, [_i32, _i32, _i64]),
     "sgl_memory_update": (ctypes.c_int, [_i32, _i32, _i32, _i64] + [_vp] * 25),
+    "sgl_memory_update_workspace_bytes": (_sz, [_i32, _i32, _i32, _i64]),
+    "sgl_memory_update_commit": (ctypes.c_int, [_i32, _i32, _i32, _i64] + [_vp] * 31 + [_sz, _vp]),
+    "sgl_memory_rows": (ctypes.c_int, [_i32, _i32, _i32, _i64] + [_vp] * 12 + [_sz, _vp]),
     "sgl_memory_update_bf16": (ctypes.c_int, [_i32, _i32, _i32, _i64] + [_vp] * 26),
     "sgl_gru_packed_elems": (_i64, [_i32, _i32]),
     "sgl_gru_pack_bf16": (ctypes.c_int, [_i32, _i32] + [_vp] * 6),

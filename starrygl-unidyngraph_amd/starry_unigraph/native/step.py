@@ -359,6 +359,7 @@ class DeviceStep:
         # HIP events around each library call, or None
         self.timer: list | None = None
         self.timed: set[str] | None = None   # names to time (None = all)
+        self._gru_ws: tuple | None = None   # (_gru_workspace(),) once asked for
         # conv_backward's weight-gradient job tables over these buffers, by form
         self._grads: tuple | None = None
         # bf16 weight copies for the attention / predictor products (Bf16Shadow), or None: fp32
@@ -461,11 +462,37 @@ class DeviceStep:
             P(b.win_dst), P(b.cnt_src), P(b.cnt_dst), P(b.new_mem),
             *([P(gru.get("packed"))] if fn == "sgl_memory_update_bf16" else []), self._s()), fn))
 
+    def _gru_workspace(self) -> torch.Tensor | None:
+        """The fp32 memory update's workspace (kept: launch plans point at it),
+        or None where the one-launch kernel serves these shapes."""
+        if self._gru_ws is None:
+            st = self.state
+            n = int(self.lib.sgl_memory_update_workspace_bytes(st.D, st.K, st.F, self.buf.cap))
+            self._gru_ws = (_capi.workspace(n, self.dev) if n > 0 else None,)
+        return self._gru_ws[0]
+
     def commit(self) -> None:
         b, st, P = self.buf, self.state, _capi.ptr
         self._call("memory_commit", lambda: _capi.check(_capi.call("sgl_memory_commit", 
             st.D, b.cap, P(b.num_roots), P(b.roots), P(b.new_mem), P(st.memory), P(st.memory_ts), P(b.ts_max),
             P(st.node_bits), P(b.hop.cnt), P(b.any_edges), P(b.root_dt), self._s()), "sgl_memory_commit"))
+
+    def update_and_commit(self, gru: dict, src, dst, efeat, ts, from_cursor: bool = False) -> None:
+        """update_memory() then commit(); small fp32 batches by
+        sgl_memory_update_commit (the same results)."""
+        ws = None if gru["w_ih"].dtype == torch.bfloat16 else self._gru_workspace()
+        if ws is None:
+            self.update_memory(gru, src, dst, efeat, ts, from_cursor=from_cursor)
+            self.commit()
+            return
+        b, st, P = self.buf, self.state, _capi.ptr
+        self._call("memory_update", lambda: _capi.check(_capi.call("sgl_memory_update_commit",
+            st.D, st.K, st.F, b.cap, P(b.num_roots), P(b.roots), P(st.memory), P(st.mailbox), P(st.mailbox_ts),
+            P(st.next_mail_pos), P(gru["w_ih"]), P(gru["w_hh"]), P(gru["b_ih"]), P(gru["b_hh"]), P(gru["wc_ih"]),
+            P(gru["wc_hh"]), P(gru["bc_ih"]), P(gru["bc_hh"]), P(src), P(dst), P(efeat), P(ts),
+            P(b.batch_start) if from_cursor else None, P(b.win_src), P(b.win_dst), P(b.cnt_src), P(b.cnt_dst),
+            P(b.new_mem), P(st.memory_ts), P(b.ts_max), P(st.node_bits), P(b.hop.cnt), P(b.any_edges), P(b.root_dt),
+            P(ws), ws.numel(), self._s()), "sgl_memory_update_commit"))
 
     def gather_memory(self) -> None:
         """The commit's place without a memory updater: the roots' memory rows
