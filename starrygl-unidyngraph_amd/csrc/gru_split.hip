@@ -36,7 +36,9 @@ constexpr int kMsgParts = 2;    // workgroups of a tile's messages
 constexpr int kMaxWidth = 512;  // S = 2D + F (so D <= 256: at most 16 column chunks)
 
 // Above this capacity the one-launch kernel has a tile for most CUs and the
-// workspace's traffic is no longer free.
+// workspace's traffic is no longer free (split against one launch, us: D 100, S
+// 372, K 1: 2,048 rows 28 / 31, 4,096 35 / 32; D 172, S 360, K 4: 117 / 132 and
+// 176 / 139; D 64, S 144, K 2: 18 / 22 and 24 / 23).
 constexpr int64_t kSplitMaxRows = 2048;
 
 struct Events {  // one batch's messages (all NULL: none are written)
