@@ -72,17 +72,21 @@ inline PlanSignal take_signal() {
 int launch_gate(const PlanGate &g, hipStream_t stream);
 int launch_signal(const PlanSignal &s, hipStream_t stream);
 
-// One thread: poll the gate word (acquire, agent scope) with s_sleep between
-// reads; after ~2 s (100 MHz clock) set the timeout word and give up.
+// One thread: poll the gate word with s_sleep between reads; after ~2 s (100
+// MHz clock) set the timeout word and give up. The polls are relaxed (an
+// acquire load invalidates the CU's and the XCD's caches, at every poll, under
+// the kernels that run beside the wait); one acquire fence (agent scope) after
+// the last of them orders what follows.
 __device__ __forceinline__ void gate_wait(const uint32_t *word, uint32_t value, uint32_t *timeout) {
   const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
-  while (__hip_atomic_load(word, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) < value) {
+  while (__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < value) {
     if (__builtin_amdgcn_s_memrealtime() - t0 > 200000000ull) {
       __hip_atomic_store(timeout, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      return;
+      break;
     }
-    __builtin_amdgcn_s_sleep(1);
+    __builtin_amdgcn_s_sleep(4);
   }
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
 }
 
 template <typename F, typename... Args>

@@ -67,15 +67,23 @@ inline size_t lds_bytes(int n_pos, int n_neg) { return sizeof(float) * std::max<
 
 __device__ __forceinline__ float sigmoid_f32(float x) { return 1.f / (1.f + expf(-x)); }
 
-template <typename T>
-__device__ __forceinline__ T block_sum(T v, T *s_part) {
-  v = sgl::wave_reduce_sum(v);
+// The workgroup's sums of three values, in every thread.
+struct Sums {
+  double v[3];
+};
+__device__ __forceinline__ Sums block_sums(Sums x, double (*s_part)[3]) {
   const int lane = threadIdx.x & (sgl::kWave - 1), w = threadIdx.x / sgl::kWave;
-  if (lane == 0) s_part[w] = v;
-  __syncthreads();
-  T t = 0;
 #pragma unroll
-  for (int i = 0; i < kBlock / sgl::kWave; ++i) t += s_part[i];
+  for (int c = 0; c < 3; ++c) {
+    x.v[c] = sgl::wave_reduce_sum(x.v[c]);
+    if (lane == 0) s_part[w][c] = x.v[c];
+  }
+  __syncthreads();
+  Sums t{};
+#pragma unroll
+  for (int i = 0; i < kBlock / sgl::kWave; ++i)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) t.v[c] += s_part[i][c];
   __syncthreads();
   return t;
 }
@@ -89,7 +97,7 @@ __device__ __forceinline__ void run(const Args &a, unsigned b, unsigned nb) {
   // with +inf, neither below nor equal to a score); cp, cn multiples of 4
   extern __shared__ float4 s_score4[];
   float *s_score = reinterpret_cast<float *>(s_score4);
-  __shared__ double s_part[kBlock / sgl::kWave];
+  __shared__ double s_part[kBlock / sgl::kWave][3];
   __shared__ bool s_last;
   const int tid = threadIdx.x;
   const int cp = ((P + kSlices - 1) / kSlices + 3) & ~3, cn = ((N + kSlices - 1) / kSlices + 3) & ~3;
@@ -144,17 +152,12 @@ __device__ __forceinline__ void run(const Args &a, unsigned b, unsigned nb) {
     gp += __shfl_xor(gp, d, sgl::kWave);
   }
   const bool lead = ip < P && slice == 0;
-  const double t_mrr = lead ? double(lt) : 0.0;
-  const double t_auc = lead ? double(lt) + 0.5 * double(eq) : 0.0;
-  const double t_ap = lead ? double(gp) / double(gp + N - lt) : 0.0;
-  const double b_mrr = block_sum(t_mrr, s_part);
-  const double b_auc = block_sum(t_auc, s_part);
-  const double b_ap = block_sum(t_ap, s_part);
+  const Sums blk = block_sums(lead ? Sums{double(lt), double(lt) + 0.5 * double(eq), double(gp) / double(gp + N - lt)}
+                                   : Sums{}, s_part);  // mrr, auc, ap
   if (tid == 0) {
     double *pp = a.partials + 3 * b;
-    pp[0] = b_mrr;
-    pp[1] = b_auc;
-    pp[2] = b_ap;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) pp[c] = blk.v[c];
     __threadfence();   // the partials before the count (release)
     s_last = atomicAdd(a.done, 1u) == nb - 1u;
   }
@@ -163,16 +166,14 @@ __device__ __forceinline__ void run(const Args &a, unsigned b, unsigned nb) {
   __threadfence();     // every workgroup's partials after its count (acquire)
   // the partials in a fixed order: thread t sums workgroups t, t + 1024, ...,
   // then a fixed tree over the threads
-  double p_mrr = 0.0, p_auc = 0.0, p_ap = 0.0;
+  Sums part{};
   for (unsigned w = tid; w < nb; w += kBlock) {
     const double *pp = a.partials + 3 * w;
-    p_mrr += pp[0];
-    p_auc += pp[1];
-    p_ap += pp[2];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) part.v[c] += pp[c];
   }
-  const double s_mrr = block_sum(p_mrr, s_part);
-  const double s_auc = block_sum(p_auc, s_part);
-  const double s_ap = block_sum(p_ap, s_part);
+  const Sums all = block_sums(part, s_part);
+  const double s_mrr = all.v[0], s_auc = all.v[1], s_ap = all.v[2];
   if (tid != 0) return;
   *a.done = 0u;
   const double nan = __longlong_as_double(0x7ff8000000000000ll);
