@@ -395,11 +395,8 @@ __global__ __launch_bounds__(kPrepBlock) void k_step_prepare_wg(
   if (blockIdx.x > 0) {
     // the workgroups past the first: a previous step's link metrics
     // (sgl_batch_prepare_metrics), which read only that step's logits and
-    // loss, after the same gate
-    if (gate_word != nullptr) {
-      if (threadIdx.x == 0) sgl::gate_wait(gate_word, gate_value, gate_timeout);
-      __syncthreads();
-    }
+    // loss. In a launch plan that entry's gate is a launch of its own, so
+    // nothing is waited for here.
     sgl::met::run(mr, blockIdx.x - 1, gridDim.x - 1);
     return;
   }
