@@ -43,6 +43,7 @@
 // No 1/sqrt(d) scaling (models.py:125). The time-encoding argument is
 // fl(fl(dt * w) + b), then cos.
 #include <climits>
+#include <type_traits>
 
 #include "common.h"
 #include "mfma.h"
@@ -67,8 +68,10 @@ constexpr int rows_for(int nw) { return nw == 16 ? 4 : 8; }
 // layouts fit in LDS (fp32_four_fits): a 16-row product tile of 4 roots costs
 // about what one of 8 does, and twice the workgroups share the step's roots
 // (config 1, 8 waves: forward 44.0 -> 37.8 us, backward 41.3 -> 33.9 us;
-// 2 roots 37.4 / 35.4). Wider shapes (config 5's 4 heads of 288 columns:
-// the merge partials need 184 KB) keep 8 roots, one wave each.
+// 2 roots 37.4 / 35.4); with several heads their 16-wave twins run where the
+// layouts fit (Split: 35.3 -> 32.3 and 31.1 -> 28.4 us). Wider shapes (config
+// 5's 4 heads of 288 columns: the merge partials need 184 KB) keep 8 roots,
+// one wave each.
 constexpr int kFp32Rows = 4;
 
 struct Dims {
@@ -1365,10 +1368,10 @@ using FwdFn = decltype(&k_conv_fwd<1, 2, false>);
 using BwdFn = decltype(&k_conv_bwd<1, 2, false>);
 // bf16 instances whose whole-head arrays need the 8-wave instances'
 // registers split each root's heads over two waves of a 16-wave workgroup,
-// keeping the 8 roots per workgroup of the 8-wave shape.
-// The fp32 products' registers do not leave room for it; the backward's
-// widest shape (4 heads, 8 column blocks) would spill over 200 bytes a lane
-// under the 16-wave register cap and keeps the 8-wave instance.
+// keeping the 8 roots per workgroup of the 8-wave shape (the fp32 ones with 4
+// roots: Split, below). The backward's widest shape (4 heads, 8 column blocks)
+// would spill over 200 bytes a lane under the 16-wave register cap and keeps
+// the 8-wave instance.
 constexpr bool split_heads(int hm, int jm) { return waves_for(hm, jm) == 8 && hm >= 2; }
 constexpr bool split_heads_bwd(int hm, int jm) { return split_heads(hm, jm) && hm * jm <= 24; }
 // fp32 and dropout instances: FwdPick / BwdPick (/ ...Drop) with kFp32Rows
@@ -1446,6 +1449,48 @@ struct BwdPickDropWide {
   static Instance<BwdFn> get() { return {&k_conv_bwd<HM, JM, true>, waves_for(HM, JM), rows_for(waves_for(HM, JM))}; }
 };
 
+// The fp32 and dropout instances with each root's heads split over the waves
+// of a 16-wave workgroup (4 roots, 2 head groups, 2 window slices), where
+// their registers do not spill under the 1024-thread cap; else no instance.
+// Such a kernel is a chain of phases (products of 16-row tiles, edge windows),
+// each as long as its waves' loads and MFMAs: 8 waves of 186 registers are two
+// a SIMD, 16 of 98 are four, every phase has twice the waves to issue from, and
+// the idle ones encode the times beside the Q product. The same slices and rows.
+//   8 waves -> split, us (forward / backward), roots of batches of
+//   B = 200, 372 columns, 2 heads:            35.3 -> 32.3 / 31.1 -> 28.4
+//   B = 3000, the same:                       65.7 -> 59.3 / 57.2 -> 51.9
+//   B = 600, 432 columns, 2 heads, 20 entries: 60.2 -> 47.5 / (45.4: spills)
+//   B = 200 / 3000, 120 columns, 4 heads:     23.1 -> 22.0, 24.4 -> 23.3 / 21.8 -> 20.9, 22.8 -> 22.4
+//   B = 600 / 3000, 216 columns, 4 heads:     37.2 -> 30.4, 46.9 -> 37.6 / 31.6 -> 27.0, 38.7 -> 33.1
+constexpr bool split_fp32(int hm, int jm) { return split_heads(hm, jm) && hm * jm <= 24; }
+constexpr bool split_fp32_bwd(int hm, int jm) { return split_heads(hm, jm) && jm <= 6 && hm * jm <= 16; }
+template <bool DROP>
+struct Split {
+  template <int HM, int JM>
+  struct Fwd {
+    static Instance<FwdFn> get() {
+      if constexpr (split_fp32(HM, JM)) return {&k_conv_fwd<HM, JM, DROP, false, 16, kFp32Rows, 2>, 16, kFp32Rows, 2};
+      else return {nullptr, 0, 0};
+    }
+  };
+  template <int HM, int JM>
+  struct Bwd {
+    static Instance<BwdFn> get() {
+      if constexpr (split_fp32_bwd(HM, JM)) return {&k_conv_bwd<HM, JM, DROP, false, 16, kFp32Rows, 2>, 16, kFp32Rows, 2};
+      else return {nullptr, 0, 0};
+    }
+  };
+};
+
+// A workgroup's dynamic LDS: the CU's less the kernels' static words.
+constexpr size_t kLdsBytes = 160 * 1024 - 512;
+template <typename Fn>
+size_t lds_bytes(const Dims &d, const Instance<Fn> &inst, int ts_rows = 0) {
+  const bool fwd = std::is_same<Fn, FwdFn>::value;
+  return sizeof(float) * (fwd ? fwd_lds_floats(d, inst.waves, inst.rows, inst.slices(), ts_rows)
+                              : bwd_lds_floats(d, inst.waves, inst.rows, inst.slices()));
+}
+
 // Whether the fp32 / dropout instances of these dimensions take kFp32Rows
 // roots: always with 16 waves (their own rows), with 8 waves when the
 // forward's (time encodings not staged) and the backward's 4-root layouts,
@@ -1457,9 +1502,13 @@ bool fp32_four_fits(const Dims &d, int nw) {
   return sizeof(float) * fwd_lds_floats(d, nw, kFp32Rows, slices, 0) <= 160 * 1024 &&
          sizeof(float) * bwd_lds_floats(d, nw, kFp32Rows, slices) <= 160 * 1024;
 }
+// The instance that runs: `four`, or its twin `split` with the same rows (so
+// the caller's per-tile arrays stay as they are) where there is one and its
+// larger layout fits, or `wide`.
 template <class Fn>
-Instance<Fn> fp32_or_wide(const Dims &d, Instance<Fn> four, Instance<Fn> (*wide)(const Dims &)) {
-  return four.fn == nullptr || fp32_four_fits(d, four.waves) ? four : wide(d);
+Instance<Fn> fp32_or_wide(const Dims &d, Instance<Fn> four, Instance<Fn> (*wide)(const Dims &), Instance<Fn> split) {
+  if (four.fn != nullptr && !fp32_four_fits(d, four.waves)) return wide(d);
+  return split.fn != nullptr && lds_bytes(d, split) <= kLdsBytes ? split : four;
 }
 
 // The bf16 weight copies' shapes (sgl_bf16_weights): every pointer set,
@@ -1540,7 +1589,8 @@ extern "C" int sgl_dropout_masks(int64_t rows, int32_t fanout, int32_t H, int32_
 extern "C" int32_t sgl_conv_tile_rows(int32_t D, int32_t F, int32_t T, int32_t H) {
   const Dims d{D, F, T, H, D + F + T, H > 0 ? D / H : 0, 0};
   if (check_dims(d) != SGL_OK) return 0;
-  const auto inst = fp32_or_wide(d, pick_instance<BwdPick>(d), &pick_instance<BwdPickWide>);
+  const auto inst = fp32_or_wide(d, pick_instance<BwdPick>(d), &pick_instance<BwdPickWide>,
+                                      pick_instance<Split<false>::Bwd>(d));
   return inst.fn != nullptr ? inst.rows : 0;
 }
 
@@ -1548,7 +1598,8 @@ extern "C" int32_t sgl_conv_backward_tile_rows(int32_t D, int32_t F, int32_t T, 
   const Dims d{D, F, T, H, D + F + T, H > 0 ? D / H : 0, 0};
   if (check_dims(d) != SGL_OK) return 0;
   const auto inst = bf16 ? pick_instance<BwdPickBf>(d)
-                         : fp32_or_wide(d, pick_instance<BwdPick>(d), &pick_instance<BwdPickWide>);
+                         : fp32_or_wide(d, pick_instance<BwdPick>(d), &pick_instance<BwdPickWide>,
+                                      pick_instance<Split<false>::Bwd>(d));
   return inst.fn != nullptr ? inst.rows : 0;
 }
 
@@ -1605,14 +1656,15 @@ extern "C" int sgl_conv_forward_passes(int32_t D, int32_t F, int32_t T, int32_t 
                   y && (fanout == 0 || (X && dt && sv_score && (T == 0 || S))),
               "conv_forward: NULL array");
   const auto inst = bw != nullptr ? pick_instance<FwdPickBf>(d)
-                    : drop ? fp32_or_wide(d, pick_instance<FwdPickDrop>(d), &pick_instance<FwdPickDropWide>)
-                           : fp32_or_wide(d, pick_instance<FwdPick>(d), &pick_instance<FwdPickWide>);
+                    : drop ? fp32_or_wide(d, pick_instance<FwdPickDrop>(d), &pick_instance<FwdPickDropWide>,
+                                      pick_instance<Split<true>::Fwd>(d))
+                           : fp32_or_wide(d, pick_instance<FwdPick>(d), &pick_instance<FwdPickWide>,
+                                      pick_instance<Split<false>::Fwd>(d));
   SGL_REQUIRE(inst.fn != nullptr, "conv_forward: no kernel instance for H=%d C=%d", H, d.C);
   // stage the tile's time encodings in LDS when they fit
-  const int slices = inst.slices();
   int ts_rows = fanout > 0 && T > 0 ? inst.rows * fanout : 0;
-  if (sizeof(float) * fwd_lds_floats(d, inst.waves, inst.rows, slices, ts_rows) > 160 * 1024) ts_rows = 0;
-  const size_t lds = sizeof(float) * fwd_lds_floats(d, inst.waves, inst.rows, slices, ts_rows);
+  if (lds_bytes(d, inst, ts_rows) > kLdsBytes) ts_rows = 0;
+  const size_t lds = lds_bytes(d, inst, ts_rows);
   SGL_REQUIRE(lds <= 160 * 1024, "conv_forward: %zu bytes of LDS needed (> 160 KiB)", lds);
   SGL_CHECK_HIP(sgl::ensure_dynamic_lds(reinterpret_cast<const void *>(inst.fn), lds));
   ConvParams p{w_q, b_q, w_k, b_k, w_v, b_v, w_out, b_out, ln_g, ln_b, te_w, te_b};
@@ -1659,15 +1711,17 @@ extern "C" int sgl_conv_backward_passes(int32_t D, int32_t F, int32_t T, int32_t
                   (fanout == 0 || (X && dt && sv_score && (T == 0 || S))),
               "conv_backward: NULL array");
   const auto inst = bw != nullptr ? pick_instance<BwdPickBf>(d)
-                    : drop ? fp32_or_wide(d, pick_instance<BwdPickDrop>(d), &pick_instance<BwdPickDropWide>)
-                           : fp32_or_wide(d, pick_instance<BwdPick>(d), &pick_instance<BwdPickWide>);
+                    : drop ? fp32_or_wide(d, pick_instance<BwdPickDrop>(d), &pick_instance<BwdPickDropWide>,
+                                      pick_instance<Split<true>::Bwd>(d))
+                           : fp32_or_wide(d, pick_instance<BwdPick>(d), &pick_instance<BwdPickWide>,
+                                      pick_instance<Split<false>::Bwd>(d));
   SGL_REQUIRE(inst.fn != nullptr, "conv_backward: no kernel instance for H=%d C=%d", H, d.C);
   // one ln_part / te_part tile per workgroup: the caller sized them by
   // sgl_conv_backward_tile_rows (the dropout instances' rows are the fp32 ones)
   const int32_t tile_rows = sgl_conv_backward_tile_rows(D, F, T, H, bw != nullptr ? 1 : 0);
   SGL_REQUIRE(inst.rows == tile_rows, "conv_backward: %d roots per workgroup, %d per tile", inst.rows, tile_rows);
   SGL_REQUIRE(npass == 1 || part_tiles >= capacity / inst.rows, "conv_backward: the passes' partials overlap");
-  const size_t lds = sizeof(float) * bwd_lds_floats(d, inst.waves, inst.rows, inst.slices());
+  const size_t lds = lds_bytes(d, inst);
   SGL_REQUIRE(lds <= 160 * 1024, "conv_backward: %zu bytes of LDS needed (> 160 KiB)", lds);
   SGL_CHECK_HIP(sgl::ensure_dynamic_lds(reinterpret_cast<const void *>(inst.fn), lds));
   ConvParams p{w_q, b_q, w_k, b_k, w_v, b_v, w_out, b_out, ln_g, ln_b, nullptr, te_b};
