@@ -6,11 +6,15 @@
 //   1. key[i] = col[i] (range-checked), val[i] = i, record[i] = (ts, row, eid)
 //   2. stable LSD radix sort of (key, val) over ceil(log2(N+1)) bits -- a
 //      stable sort keyed by dst keeps event order inside each node's list
+//      (val as a counting iterator: the sort writes it out itself, 9 us more
+//      for 7 saved in step 1)
 //   3. gather the records through the sorted event index (int32 / int64 SoA):
 //      the event order inside a list is random to the memory system, so an
 //      event costs one 128-byte line as a record and one per array otherwise
 //      (7.8 M events, 1.1 M nodes: 293 -> 162 us; writing the records adds 20)
-//   4. indptr from the boundaries of the sorted keys (no atomics)
+//   4. indptr from the boundaries of the sorted keys (no atomics), by the
+//      gather's threads: its lines bound that kernel, and the keys' few more
+//      bytes mostly hide behind them (163.3 + 23.8 us apart, 168.6 together)
 #include <rocprim/device/device_radix_sort.hpp>
 
 #include <climits>
@@ -67,26 +71,32 @@ __global__ __launch_bounds__(kBlock) void k_tcsr_keys(
   rec[i] = EventRecord{ts[i], int32_t(s), int32_t(id)};
 }
 
-__global__ __launch_bounds__(kBlock) void k_tcsr_gather(
-    int64_t num_edges, const int32_t *__restrict__ order, const EventRecord *__restrict__ rec,
-    int32_t *__restrict__ nbr, int32_t *__restrict__ eid_out, int64_t *__restrict__ ts_out) {
-  const int64_t j = int64_t(blockIdx.x) * kBlock + threadIdx.x;
-  if (j >= num_edges) return;
-  const EventRecord r = rec[order[j]];  // order: a permutation of [0, num_edges)
-  nbr[j] = r.row;
-  eid_out[j] = r.eid;
-  ts_out[j] = r.ts;
-}
-
 // Thread j in [0, E] writes indptr[n] = j for every node n in (key[j-1], key[j]].
-__global__ __launch_bounds__(kBlock) void k_tcsr_indptr(
-    int64_t num_edges, int64_t num_nodes, const uint32_t *__restrict__ skeys,
-    int64_t *__restrict__ indptr) {
-  const int64_t j = int64_t(blockIdx.x) * kBlock + threadIdx.x;
-  if (j > num_edges) return;
+__device__ __forceinline__ void write_indptr(int64_t j, int64_t num_edges, int64_t num_nodes,
+                                             const uint32_t *__restrict__ skeys, int64_t *__restrict__ indptr) {
   const int64_t prev = j == 0 ? -1 : int64_t(skeys[j - 1]);
   const int64_t cur = j == num_edges ? num_nodes : int64_t(skeys[j]);
   for (int64_t n = prev + 1; n <= cur && n <= num_nodes; ++n) indptr[n] = j;
+}
+
+__global__ __launch_bounds__(kBlock) void k_tcsr_gather(
+    int64_t num_edges, int64_t num_nodes, const int32_t *__restrict__ order, const uint32_t *__restrict__ skeys,
+    const EventRecord *__restrict__ rec, int32_t *__restrict__ nbr, int32_t *__restrict__ eid_out,
+    int64_t *__restrict__ ts_out, int64_t *__restrict__ indptr) {
+  const int64_t j = int64_t(blockIdx.x) * kBlock + threadIdx.x;
+  if (j > num_edges) return;
+  if (j < num_edges) {
+    const EventRecord r = rec[order[j]];  // order: a permutation of [0, num_edges)
+    nbr[j] = r.row;
+    eid_out[j] = r.eid;
+    ts_out[j] = r.ts;
+  }
+  write_indptr(j, num_edges, num_nodes, skeys, indptr);
+}
+
+__global__ __launch_bounds__(kBlock) void k_tcsr_indptr(int64_t num_nodes, int64_t *__restrict__ indptr) {  // no edges
+  const int64_t n = int64_t(blockIdx.x) * kBlock + threadIdx.x;
+  if (n <= num_nodes) indptr[n] = 0;
 }
 
 // The sampler's packed copy of a CSR: int32 times, (nbr, eid) pairs and every
@@ -192,13 +202,12 @@ extern "C" int sgl_tcsr_build(int64_t num_nodes, int64_t num_edges,
                                              err_flag);
     SGL_CHECK_LAUNCH();
     SGL_CHECK_HIP(rocprim::radix_sort_pairs(temp_ptr, temp, keys_in, keys_out, vals_in, vals_out, e, 0u, bits, stream));
-    k_tcsr_gather<<<grid, kBlock, 0, stream>>>(num_edges, vals_out, rec, nbr, eid_out, ts_out);
-    SGL_CHECK_LAUNCH();
     const unsigned grid1 = unsigned((e + 1 + kBlock - 1) / kBlock);
-    k_tcsr_indptr<<<grid1, kBlock, 0, stream>>>(num_edges, num_nodes, keys_out, indptr);
+    k_tcsr_gather<<<grid1, kBlock, 0, stream>>>(num_edges, num_nodes, vals_out, keys_out, rec, nbr, eid_out, ts_out,
+                                                indptr);
     SGL_CHECK_LAUNCH();
   } else {
-    k_tcsr_indptr<<<1, kBlock, 0, stream>>>(0, num_nodes, nullptr, indptr);
+    k_tcsr_indptr<<<unsigned((num_nodes + 1 + kBlock - 1) / kBlock), kBlock, 0, stream>>>(num_nodes, indptr);
     SGL_CHECK_LAUNCH();
   }
   return SGL_OK;
