@@ -708,7 +708,7 @@ int sgl_adam_advance(float *step, const int32_t *active, hipStream_t stream);
  *           ceil(*num_roots / -r_fixed) when r_fixed <= -2 (per-tile partial
  *           sums of tiles of -r_fixed roots: the tiles holding live roots);
  *           npass 0 counts as 1 (the passes of a dropout step). s1 >= rows
- *           (s2 may be 0: a broadcast row). Tiles: ceil(rows/16) *
+ *           (s2 may be 0: a broadcast row); s1, s2 <= 2^21. Tiles: ceil(rows/16) *
  *           ceil(cols/16), tiles_b = ceil(cols/16); the job's tile l is the
  *           16x16 block (l / tiles_b, l % tiles_b).
  *   kind 1: rows*cols contiguous elements from off whose gradient is already

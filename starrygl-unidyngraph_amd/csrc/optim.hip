@@ -89,6 +89,11 @@ namespace {
 
 constexpr int kGaBlock = 256;
 constexpr int kGaChunk = 16;  // MFMA row groups per wave per load batch
+constexpr int kGaRound = 4 * 4 * kGaChunk;  // rows of the four waves' load batches
+// Floats of a strided operand addressed from one base: with the rows that the
+// last round reads past them (masked by the range) below 2^30, 4 GiB of bytes,
+// for rows of up to 2^21 floats.
+constexpr uint64_t kGaSegFloats = 1ull << 29;
 
 struct AdamSegs {
   float *step[SGL_MAX_ADAM_SEGMENTS];
@@ -182,24 +187,34 @@ __global__ __launch_bounds__(kGaBlock) void k_grad_adam(const sgl_grad_job *__re
     const int i16 = lane & 15, q = lane >> 4;
     sgl::f32x4 acc = {0.f, 0.f, 0.f, 0.f};
     const int npass = jb.npass > 0 ? jb.npass : 1;
-    for (int ps = 0; R > 0 && ps < npass; ++ps) {
-      // rows >= R read 0 through the buffer ranges (X1 rows are at least
-      // `rows` wide, so row R starts past X1's span)
-      const uint32_t span1 = uint32_t(R - 1) * uint32_t(jb.s1) + uint32_t(jb.rows);
-      const uint32_t span2 = uint32_t(R - 1) * uint32_t(jb.s2) + uint32_t(jb.cols);
-      const __amdgpu_buffer_rsrc_t r1 = sgl::weight_rsrc(jb.x1 + ps * jb.ps1, span1);
-      const __amdgpu_buffer_rsrc_t r2 = sgl::weight_rsrc(jb.x2 + ps * jb.ps2, span2);
-      const int ngroups = (R + 3) >> 2;
-      for (int gb = wave; gb < ngroups; gb += 4 * kGaChunk) {
-        float xa[kGaChunk], xb[kGaChunk];
+    // Buffer offsets are 32-bit bytes: rows that reach further are taken in
+    // segments, each from its own base, of whole rounds of the four waves
+    // (the same rows to the same wave in the same order as in one segment).
+    int seg = R;
+    const uint64_t widest = uint64_t(max(jb.s1, jb.s2));
+    if (uint64_t(max(R, 0)) * widest >= kGaSegFloats)  // never at a step's usual sizes
+      seg = max(kGaRound, int(kGaSegFloats / widest) & -kGaRound);
+    for (int ps = 0; ps < npass; ++ps) {
+      for (int rs = 0; rs < R; rs += seg) {
+        // rows >= n read 0 through the buffer ranges (X1 rows are at least
+        // `rows` wide, so row n starts past X1's span)
+        const int n = min(seg, R - rs);
+        const uint32_t span1 = uint32_t(n - 1) * uint32_t(jb.s1) + uint32_t(jb.rows);
+        const uint32_t span2 = uint32_t(n - 1) * uint32_t(jb.s2) + uint32_t(jb.cols);
+        const __amdgpu_buffer_rsrc_t r1 = sgl::weight_rsrc(jb.x1 + ps * jb.ps1 + rs * jb.s1, span1);
+        const __amdgpu_buffer_rsrc_t r2 = sgl::weight_rsrc(jb.x2 + ps * jb.ps2 + rs * jb.s2, span2);
+        const int ngroups = (n + 3) >> 2;
+        for (int gb = wave; gb < ngroups; gb += 4 * kGaChunk) {
+          float xa[kGaChunk], xb[kGaChunk];
 #pragma unroll
-        for (int c = 0; c < kGaChunk; ++c) {
-          const uint32_t r = uint32_t(4 * (gb + 4 * c) + q);
-          xa[c] = sgl::buf_load(r1, r * uint32_t(jb.s1) + uint32_t(a0 + i16));
-          xb[c] = sgl::buf_load(r2, r * uint32_t(jb.s2) + uint32_t(b0 + i16));
+          for (int c = 0; c < kGaChunk; ++c) {
+            const uint32_t r = uint32_t(4 * (gb + 4 * c) + q);
+            xa[c] = sgl::buf_load(r1, r * uint32_t(jb.s1) + uint32_t(a0 + i16));
+            xb[c] = sgl::buf_load(r2, r * uint32_t(jb.s2) + uint32_t(b0 + i16));
+          }
+#pragma unroll
+          for (int c = 0; c < kGaChunk; ++c) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[c], xb[c], acc, 0, 0, 0);
         }
-#pragma unroll
-        for (int c = 0; c < kGaChunk; ++c) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[c], xb[c], acc, 0, 0, 0);
       }
     }
 #pragma unroll

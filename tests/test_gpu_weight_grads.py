@@ -62,3 +62,34 @@ def test_weight_grads_match_float64_products(gpu, D, F, T, H, U, pa):
         assert bool(((x.double() - want).abs() <= (U + 8) * 2.0 ** -24 * size).all()), i
     if U == 0:
         assert all(bool((x == 0).all()) for x in got2)
+
+
+@pytest.mark.parametrize("R,s1,s2", [(1100, 40, 1 << 20), (1025, 1 << 20, 24), (1026, (1 << 20) + 3, 1 << 20)])
+def test_rows_past_32_bit_offsets(gpu, R, s1, s2):
+    """Operands that span more than 4 GiB (rows far apart stand for many rows): the same bits as from compact copies."""
+    from starry_unigraph.lib import _capi
+    rows, cols = 20, 17
+    g = torch.Generator().manual_seed(R)
+    x = [torch.randn(R, w, generator=g).to(gpu) for w in (rows, cols)]
+
+    def spread(t, stride):
+        out = torch.zeros(R, stride, device=gpu)
+        out[:, :t.shape[1]] = t
+        return out
+
+    n = torch.tensor([R], dtype=torch.int32, device=gpu)
+    tiles = torch.arange(4, dtype=torch.int32, device=gpu) * 256
+    got = []
+    for a, b in ((s1, s2), (32, 32)):
+        x1, x2 = spread(x[0], a), spread(x[1], b)
+        job = _capi.GradJob(x1=x1.data_ptr(), x2=x2.data_ptr(), s1=a, s2=b, off=0, ldo=cols, rows=rows, cols=cols,
+                            kind=0, r_fixed=-1, tiles_b=2, npass=1)
+        raw = torch.frombuffer(bytearray(bytes(job)), dtype=torch.uint8).to(gpu)
+        out = torch.empty(rows, cols, device=gpu)
+        _capi.check(_capi.lib().sgl_weight_grads(raw.data_ptr(), tiles.data_ptr(), 4, n.data_ptr(), out.data_ptr(),
+                                                 _capi.stream_of(gpu)), "sgl_weight_grads")
+        got.append(out.clone())
+        del x1, x2
+    assert torch.equal(*got)
+    size = x[0].abs().double().T @ x[1].abs().double()
+    assert bool(((got[0].double() - x[0].double().T @ x[1].double()).abs() <= (R + 8) * 2.0 ** -24 * size).all())
