@@ -632,12 +632,16 @@ class DeviceStep:
 
     def conv_backward(self, params: list[torch.Tensor], efeat_all: torch.Tensor, gy: torch.Tensor, drop=None):
         """The backward kernel and the weight gradients (the autograd path,
-        one pass; sgl_weight_grads, no host synchronisation). Returns the 12
-        parameter gradients (TimeEncode w, b; w_q, b_q, w_k, b_k, w_v, b_v,
-        w_out, b_out, ln weight, ln bias), views of one new buffer."""
+        one pass): by sgl_weight_grads without a host synchronisation, or for
+        many roots (weight_grads_in_one_launch) as torch products over the live
+        rows. Returns the 12 parameter gradients (TimeEncode w, b; w_q, b_q,
+        w_k, b_k, w_v, b_v, w_out, b_out, ln weight, ln bias), of the first in
+        views of one new buffer."""
         self.conv_backward_kernel(params, efeat_all, gy, drop=drop)
         att_drop = drop is not None and drop[0] > 0
         key = (att_drop, self.bwd_tile_rows(self.bf16 is not None and drop is None))
+        if not weight_grads_in_one_launch(self.buf.cap, self.dims.D, self.dims.C):
+            return self._weight_grad_products(params, *key)
         if self._grads is None or self._grads[0] is not self.buf:
             self._grads = (self.buf, {})
         jobs, table, tiles, sizes = (self._grads[1].get(key) or self._weight_grad_jobs(params, *key))[:4]
@@ -646,6 +650,30 @@ class DeviceStep:
         self._call("weight_grads", lambda: _capi.check(_capi.call(
             "sgl_weight_grads", jobs, table, tiles, P(self.buf.num_roots), P(flat), self._s()), "sgl_weight_grads"))
         return [g.view(p.shape) for g, p in zip(flat.split_with_sizes(sizes), params)]
+
+    def _weight_grad_products(self, params: list[torch.Tensor], att_drop: bool, tile_rows: int) -> list[torch.Tensor]:
+        """conv_backward's weight gradients as torch products over the live
+        root rows (one host read of their number; the kernels leave the rows
+        past them unwritten)."""
+        b, d = self.buf, self.dims
+        D, H, C, T = d.D, d.H, d.C, d.T
+        dh = D // H
+        c = int(b.num_roots.item())
+        gz, gagg, gQ, new_mem = b.gz[:c], b.gagg[:c], b.gQ[:c], b.new_mem[:c]
+        ga, qh = gagg.reshape(c, H, dh), b.Q[:c].reshape(c, H, dh)
+
+        def per_head(x, rows):   # [c, H, dh], [c, H, C] -> [D, C]
+            return torch.bmm(x.permute(1, 2, 0).contiguous(), rows[:c].permute(1, 0, 2).contiguous()).reshape(D, C)
+
+        w_q = torch.cat([gQ.t() @ new_mem, torch.outer(gQ.sum(0), torch.cos(params[1]))], dim=1)
+        w_out = torch.cat([gz.t() @ b.agg[:c], gz.t() @ new_mem], dim=1)
+        # with attention dropout the kept weights sum to s_h, not 1
+        b_v = (ga * b.sdrop[:c].unsqueeze(-1)).sum(0).reshape(D) if att_drop else gagg.sum(0)
+        b_k = (qh * b.sigma[:c].unsqueeze(-1)).sum(0).reshape(D)
+        nt = b.cap // tile_rows
+        te, ln = b.te_part[:nt, :, :T].sum(0), b.ln_part[:nt].sum(0)
+        return [te[0].reshape(T, 1), te[1], w_q, gQ.sum(0), per_head(qh, b.G), b_k, per_head(ga, b.xbar), b_v, w_out,
+                gz.sum(0), ln[0], ln[1]]
 
     def _weight_grad_jobs(self, params: list[torch.Tensor], att_drop: bool, tile_rows: int) -> tuple:
         """sgl_weight_grads' job and tile tables over this step's buffers (device
@@ -669,6 +697,22 @@ class DeviceStep:
         at = raw.data_ptr()
         made = self._grads[1][att_drop, tile_rows] = (at, at + ctypes.sizeof(arr), table.numel(), sizes, raw, one)
         return made
+
+
+# Root rows x D x C above which sgl_weight_grads is not the faster way.
+GRAD_LAUNCH_MAX = 3 << 30
+
+
+def weight_grads_in_one_launch(rows: int, D: int, C: int) -> bool:
+    """Whether conv_backward takes its weight gradients from sgl_weight_grads
+    for step buffers of ``rows`` roots. Its workgroups each walk every row of
+    a 16x16 block, and each strip of X is read by D / 16 of them, so rows x D x
+    C sets its time, where a matrix product splits the rows. One launch against
+    products, us, at 8,192 / 65,536 / 131,072 rows: D 100, C 372, two heads
+    104 / 390, 1,279 / 1,748, 2,927 / 2,728; D 172, C 288, four heads 185 / 407,
+    1,980 / 1,975, 4,332 / 3,032 (the two meet at 65,536: 3.2e9); D 64, C 120,
+    four heads 44 / 391, 380 / 1,188, 755 / 2,166."""
+    return rows * D * C <= GRAD_LAUNCH_MAX
 
 
 def attention_grad_jobs(b: "StepBuffers", d: "ConvDims", off, one: int, gemm, tile_rows: int, att_drop: bool,

@@ -64,6 +64,17 @@ def test_weight_grads_match_float64_products(gpu, D, F, T, H, U, pa):
         assert all(bool((x == 0).all()) for x in got2)
 
 
+@pytest.mark.parametrize("D,F,T,H,U,pa", [(30, 5, 7, 3, 15, 0.0), (44, 1, 20, 4, 17, 0.3), (32, 6, 16, 2, 0, 0.0)])
+def test_products_for_many_roots(gpu, monkeypatch, D, F, T, H, U, pa):
+    """The other side of weight_grads_in_one_launch, the same check."""
+    from starry_unigraph.native import step
+    assert step.weight_grads_in_one_launch(65536, 100, 372)
+    assert not step.weight_grads_in_one_launch(131072, 100, 372) and not step.weight_grads_in_one_launch(131072, 172, 288)
+    monkeypatch.setattr(step, "GRAD_LAUNCH_MAX", 0)
+    monkeypatch.setattr(step.DeviceStep, "_weight_grad_jobs", None)   # (not reached)
+    test_weight_grads_match_float64_products(gpu, D, F, T, H, U, pa)
+
+
 @pytest.mark.parametrize("R,s1,s2", [(1100, 40, 1 << 20), (1025, 1 << 20, 24), (1026, (1 << 20) + 3, 1 << 20)])
 def test_rows_past_32_bit_offsets(gpu, R, s1, s2):
     """Operands that span more than 4 GiB (rows far apart stand for many rows): the same bits as from compact copies."""
