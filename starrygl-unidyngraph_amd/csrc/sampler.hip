@@ -338,13 +338,19 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_tiles(
 // Calls body(q, j, o) for every entry j of every query q < nq of this
 // workgroup's kTile queries, o its place in the concatenated output. Threads
 // walk the tile's padded slots (q, j < k), so that the padded rows are read and
-// the output written in order; the slot's query comes from adding, not from a
-// search of the tile's offsets. Bound by the bytes: 2 M entries (40 read and
-// written each) take 29 us. With the offsets scanned once and src_index /
-// delta_ts written by k_block_index (tensor operations before: a second scan,
-// repeat_interleave and two gathers a call), two hops of 20 from 8,000 queries
-// with their four getters take 140 us of kernels and 19 launches, before 244
-// us and 52: 380 -> 169 us with the host's part.
+// the output written in order, the slot's query from adding; or, where fewer
+// than one slot in kSparse holds an entry, the entries, their queries from a
+// search of the tile's offsets (k slots a query would be walked for a few
+// entries). With the offsets scanned once and src_index / delta_ts written by
+// k_block_index (tensor operations before: a second scan, repeat_interleave
+// and two gathers a call), two hops of 20 from 8,000 queries, nearly full
+// windows, with their four getters take 140 us of kernels and 19 launches,
+// before 244 us and 52: 380 -> 169 us with the host's part; the copy there is
+// bound by its bytes (2 M entries, 40 read and written each: 29 us). Copy by
+// slots / by entries, us, 8,000 queries of 100 slots: full 46 / 93, half 36 /
+// 46, a quarter 34 / 25, an eighth 30 / 14, 1 in 100 24 / 6; of 1,000 slots a
+// quarter 261 / 288, an eighth 178 / 141, 1 in 100 106 / 12.
+constexpr int kSparse = 4;
 template <class Body>
 __device__ __forceinline__ void for_tile_entries(int64_t nq, int k, const int64_t *__restrict__ ptr, Body body) {
   __shared__ int32_t s_off[kTile + 1];
@@ -355,6 +361,18 @@ __device__ __forceinline__ void for_tile_entries(int64_t nq, int k, const int64_
   if (tid <= nt) s_off[tid] = int32_t(ptr[q0 + tid] - base);
   if (tid == 0) s_off[nt] = int32_t(ptr[q0 + nt] - base);
   __syncthreads();
+  const int total = s_off[nt];
+  if (int64_t(total) * kSparse < int64_t(nt) * k) {
+    for (int e = tid; e < total; e += kTile) {
+      int lo = 0, hi = nt;  // the entry's query: the largest q with s_off[q] <= e
+      while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (s_off[mid] <= e) lo = mid; else hi = mid;
+      }
+      body(q0 + lo, e - s_off[lo], base + e);
+    }
+    return;
+  }
   const int dq = kTile / k, dj = kTile - dq * k;
   int q = tid / k, j = tid - q * k;
   while (q < nt) {

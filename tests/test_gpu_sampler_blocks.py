@@ -49,3 +49,33 @@ def test_error_bits_come_with_the_total(gpu):
     assert bits != 0 and hops[0].count() == 1
     with pytest.raises(RuntimeError, match="node id out of range"):
         s.err.raise_if_set("sample")
+
+
+@pytest.mark.parametrize("nq,k", [(1, 4096), (300, 4096), (513, 400), (600, 9)])
+@pytest.mark.parametrize("most", [1, 3, "quarter", "one full"])
+def test_concatenated_hop_of_short_windows(gpu, nq, k, most):
+    """Windows far below the fanout (an entry walk), tiles of both kinds beside each other, and the count at which a
+    tile changes from one to the other."""
+    from starry_unigraph.native.tcsr import PaddedHop, RecentSampler, build_tcsr
+    g = torch.Generator(gpu).manual_seed(nq + k)
+    z = torch.zeros(2, dtype=torch.int64, device=gpu)
+    s = RecentSampler(build_tcsr(2, z, z, None, z))
+    if most == "quarter":   # a tile's total around a quarter of its slots
+        cnt = torch.full((nq,), k // 4, device=gpu)
+        cnt[:256] += (torch.arange(min(nq, 256), device=gpu) % 4 < k % 4).long()
+        cnt[256:257] -= 1
+    else:
+        cnt = torch.randint(0, (1 if most == "one full" else most) + 1, (nq,), generator=g, device=gpu)
+        if most == "one full":
+            cnt[nq // 2] = k
+    cnt = cnt.to(torch.int32)
+    val = lambda: torch.randint(0, 2 ** 31 - 1, (nq * k,), generator=g, device=gpu)
+    hop = PaddedHop(cnt, val().int(), val().int(), torch.rand(nq * k, generator=g, device=gpu), val(), val()[:nq], k)
+    c = s.compact(hop)
+    live = (torch.arange(k, device=gpu).unsqueeze(0) < cnt.unsqueeze(1)).reshape(-1)
+    for name in ("nbr", "eid", "dt", "ts"):
+        assert torch.equal(getattr(c, name), getattr(hop, name)[live]), name
+    q = torch.arange(nq, device=gpu).repeat_interleave(k)[live]
+    assert torch.equal(c.index("query"), q)
+    assert torch.equal(c.index("delta"), hop.q_ts[q] - hop.ts[live])
+    assert torch.equal(c.index("place"), torch.arange(k, device=gpu).repeat(nq)[live].float())
