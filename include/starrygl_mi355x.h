@@ -163,7 +163,7 @@ int sgl_recent_fill(int64_t num_queries, int32_t fanout, const int64_t *ptr,
 /* Per entry o of query q's window [ptr[q], ptr[q+1]) of a concatenated hop:
  * index[o] = q, delta[o] = q_ts[q] - ts[o], place[o] = o - ptr[q] (each may be
  * NULL; TemporalGraphBlock's src_index, delta_ts and sample_weight,
- * output.h:4-30). No window is longer than fanout. */
+ * output.h:4-30). No window is longer than fanout (0: not known). */
 int sgl_block_index(int64_t num_queries, int32_t fanout, const int64_t *ptr,
                     const int64_t *q_ts, const int64_t *ts, int64_t *index,
                     int64_t *delta, float *place, hipStream_t stream);

@@ -341,7 +341,7 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_tiles(
 // the output written in order, the slot's query from adding; or, where fewer
 // than one slot in kSparse holds an entry, the entries, their queries from a
 // search of the tile's offsets (k slots a query would be walked for a few
-// entries). With the offsets scanned once and src_index / delta_ts written by
+// entries; k 0: a window can have any length). With the offsets scanned once and src_index / delta_ts written by
 // k_block_index (tensor operations before: a second scan, repeat_interleave
 // and two gathers a call), two hops of 20 from 8,000 queries, nearly full
 // windows, with their four getters take 140 us of kernels and 19 launches,
@@ -362,7 +362,7 @@ __device__ __forceinline__ void for_tile_entries(int64_t nq, int k, const int64_
   if (tid == 0) s_off[nt] = int32_t(ptr[q0 + nt] - base);
   __syncthreads();
   const int total = s_off[nt];
-  if (int64_t(total) * kSparse < int64_t(nt) * k) {
+  if (k == 0 || int64_t(total) * kSparse < int64_t(nt) * k) {
     for (int e = tid; e < total; e += kTile) {
       int lo = 0, hi = nt;  // the entry's query: the largest q with s_off[q] <= e
       while (hi - lo > 1) {
@@ -621,7 +621,7 @@ extern "C" int sgl_recent_fill(int64_t num_queries, int32_t fanout, const int64_
 extern "C" int sgl_block_index(int64_t num_queries, int32_t fanout, const int64_t *ptr, const int64_t *q_ts,
                                const int64_t *ts, int64_t *index, int64_t *delta, float *place, hipStream_t stream) {
   SGL_REQUIRE(num_queries >= 0 && fanout >= 0 && fanout <= 4096, "block_index: bad sizes");
-  if (num_queries == 0 || fanout == 0) return SGL_OK;
+  if (num_queries == 0) return SGL_OK;
   SGL_REQUIRE(ptr != nullptr && (delta == nullptr || (q_ts && ts)), "block_index: NULL array");
   const size_t tiles = (size_t(num_queries) + kTile - 1) / kTile;
   SGL_REQUIRE(tiles < size_t(INT_MAX), "block_index: too many queries");

@@ -65,7 +65,7 @@ class SampleHop:
     dt: torch.Tensor               # float32 [M]
     ts: torch.Tensor | None        # int64 [M]
     q_ts: torch.Tensor             # int64 [Q]
-    fanout: int                    # the longest a window can be
+    fanout: int = 0                # the longest a window can be (0: not known)
 
     @property
     def num_queries(self) -> int:

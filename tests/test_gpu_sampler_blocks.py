@@ -79,3 +79,18 @@ def test_concatenated_hop_of_short_windows(gpu, nq, k, most):
     assert torch.equal(c.index("query"), q)
     assert torch.equal(c.index("delta"), hop.q_ts[q] - hop.ts[live])
     assert torch.equal(c.index("place"), torch.arange(k, device=gpu).repeat(nq)[live].float())
+
+
+def test_hop_of_unknown_fanout(gpu):
+    """A SampleHop made from its six arrays alone: windows of any length, one longer than any fanout."""
+    from starry_unigraph.native.tcsr import SampleHop
+    cnt = torch.tensor([0, 3, 1, 9000, 0, 2] + [1] * 300, device=gpu)
+    ptr = torch.cat([torch.zeros(1, dtype=torch.int64, device=gpu), cnt.cumsum(0)])
+    m = int(cnt.sum())
+    i32, ts = torch.arange(m, dtype=torch.int32, device=gpu), torch.arange(m, device=gpu) * 3
+    q_ts = torch.arange(cnt.numel(), device=gpu) * 7 + 10 ** 6
+    hop = SampleHop(ptr, i32, i32, i32.float(), ts, q_ts)
+    q = torch.arange(cnt.numel(), device=gpu).repeat_interleave(cnt)
+    assert torch.equal(hop.index("query"), q)
+    assert torch.equal(hop.index("delta"), q_ts[q] - ts)
+    assert torch.equal(hop.index("place"), (torch.arange(m, device=gpu) - ptr[q]).float())
