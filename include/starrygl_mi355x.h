@@ -507,9 +507,10 @@ int sgl_conv_backward(int32_t D, int32_t F, int32_t T, int32_t H,
  * hold npass consecutive blocks of one pass's size, pass p's output starts at
  * y + p * y_pass_stride. In the backward the gradient arrays and acc_src /
  * g_src [npass][capacity+1][D] hold such blocks too, ln_part / te_part blocks
- * of part_tiles tiles; acc_dst and gy are NULL, pass 0's dL/dy comes through
- * w_s and every other pass's through w_d (the src, dst and negative roles of
- * runtime.py:193-195). npass 1 is the single-pass call. */
+ * of part_tiles tiles; gy is every pass's dL/dy, or NULL: then acc_dst is NULL
+ * and pass 0's dL/dy comes through w_s, every other pass's through w_d (the
+ * src, dst and negative roles of runtime.py:193-195). npass 1 is the
+ * single-pass call. */
 int sgl_conv_forward_passes(int32_t D, int32_t F, int32_t T, int32_t H,
                      int32_t fanout, int64_t capacity,
                      const int32_t *num_roots, const int32_t *any_edges,

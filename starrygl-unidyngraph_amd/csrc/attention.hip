@@ -875,14 +875,16 @@ __global__ __launch_bounds__(NW * 64) void k_conv_bwd(
   if constexpr (DROP) {
     // grid row p: dropout pass dc.pass + p, its own accumulator, saved state
     // and gradients (the first pass's gradient comes through src_fc, the
-    // others' through dst_fc)
+    // others' through dst_fc; a given gy is every pass's)
     const int pass = blockIdx.y;
     if (pass > 0) {
       const size_t cap = size_t(gridDim.x) * RPW, rows = cap * pass;
       to_pass(sv, d, cap, pass);
-      acc_src += pass * (cap + 1) * D;
-      g_src += pass * (cap + 1) * D;
-      w_s = w_d;
+      if (gy == nullptr) {
+        acc_src += pass * (cap + 1) * D;
+        g_src += pass * (cap + 1) * D;
+        w_s = w_d;
+      }
       g.gz += rows * D;
       g.gagg += rows * D;
       g.gQ += rows * D;
@@ -1695,8 +1697,8 @@ extern "C" int sgl_conv_backward_passes(int32_t D, int32_t F, int32_t T, int32_t
   sgl::DropCfg dc;
   bool drop;
   if (int rc = drop_cfg(p_att, p_out, seed, rng_step, pass, sv_sdrop, dc, drop)) return rc;
-  SGL_REQUIRE(npass == 1 || (drop && npass > 1 && npass <= kMaxPasses && gy == nullptr && acc_dst == nullptr && w_d),
-              "conv_backward: %d passes (1, or up to %d with dropout, from one accumulator each)", npass, kMaxPasses);
+  SGL_REQUIRE(npass == 1 || (drop && npass > 1 && npass <= kMaxPasses && (gy || (acc_dst == nullptr && w_d))),
+              "conv_backward: %d passes (1, or up to %d with dropout, from gy or one accumulator each)", npass, kMaxPasses);
   if (bw != nullptr) {
     if (int rc = check_bf16_weights(d, *bw, drop)) return rc;
     SGL_REQUIRE(gy != nullptr || acc_dst != nullptr, "conv_backward: the bf16 products need both accumulators");

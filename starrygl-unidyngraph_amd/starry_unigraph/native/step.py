@@ -597,9 +597,9 @@ class DeviceStep:
         in the step buffers (the weight gradients are StepParamUpdate's).
         dL/dy is ``gy``, or (gy None) comes from the predictor's per-root rows
         with ``pred_w`` = (src_fc.weight, dst_fc.weight). With ``drop`` (the
-        forward's) every pass runs: pass 0 takes dL/dy from the src rows and
-        src_fc, pass 1 from the dst rows and dst_fc, pass 2 from the
-        negatives' rows and dst_fc."""
+        forward's) every pass runs: with ``gy`` for dL/dy, or pass 0 takes it
+        from the src rows and src_fc, pass 1 from the dst rows and dst_fc,
+        pass 2 from the negatives' rows and dst_fc."""
         b, d, P = self.buf, self.dims, _capi.ptr
         te_w, te_b, w_q, b_q, w_k, b_k, w_v, b_v, w_out, b_out, ln_g, ln_b = params
         hop = b.hop
@@ -607,8 +607,6 @@ class DeviceStep:
         several = drop is not None and b.passes > 1   # every pass in one launch
         acc_a = acc_b = g_a = g_b = w_a = w_b = None
         if gy is not None:
-            if several:
-                raise RuntimeError("conv_backward_kernel: the dropout passes take dL/dy from the predictor's rows")
             gy = gy.contiguous()
         elif several:
             acc_a, g_a = b.acc_all, b.g_all
@@ -632,7 +630,7 @@ class DeviceStep:
 
     def conv_backward(self, params: list[torch.Tensor], efeat_all: torch.Tensor, gy: torch.Tensor, drop=None):
         """The backward kernel and the weight gradients (the autograd path,
-        one pass): by sgl_weight_grads without a host synchronisation, or for
+        one pass; pass 0's of buffers with several): by sgl_weight_grads without a host synchronisation, or for
         many roots (weight_grads_in_one_launch) as torch products over the live
         rows. Returns the 12 parameter gradients (TimeEncode w, b; w_q, b_q,
         w_k, b_k, w_v, b_v, w_out, b_out, ln weight, ln bias), of the first in

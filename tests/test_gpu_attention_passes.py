@@ -40,7 +40,7 @@ def _step(gpu, D, F, T, H, k, U, edges, seed):
     return step, params, r(E, F), (r(D, D), r(D, D))
 
 
-def _one_at_a_time(step, params, pred_w, drop):
+def _one_at_a_time(step, params, pred_w, drop, gy=None):
     from starry_unigraph.lib import _capi
     b, d, P = step.buf, step.dims, _capi.ptr
     te_w, te_b, w_q, b_q, w_k, b_k, w_v, b_v, w_out, b_out, ln_g, ln_b = (P(t) for t in params)
@@ -62,8 +62,9 @@ def _one_at_a_time(step, params, pred_w, drop):
         _capi.check(_capi.call(
             "sgl_conv_backward", d.D, d.F, d.T, d.H, d.fanout, b.cap, P(b.num_roots), P(b.any_edges), P(b.hop.cnt),
             P(b.X), P(b.S), P(b.hop.dt), w_q, b_q, w_k, b_k, w_v, b_v, w_out, b_out, ln_g, ln_b, te_b, at(b.Q, p),
-            at(b.qt, p), at(b.xbar, p), at(b.score, p), at(b.ml, p), at(b.agg, p), at(b.z, p), at(b.stats, p), None,
-            at(b.acc_all, p), None, P(pred_w[0 if p == 0 else 1]), None, at(b.g_all, p), None, at(b.gz, p),
+            at(b.qt, p), at(b.xbar, p), at(b.score, p), at(b.ml, p), at(b.agg, p), at(b.z, p), at(b.stats, p), P(gy),
+            *((None,) * 6 if gy is not None else
+              (at(b.acc_all, p), None, P(pred_w[0 if p == 0 else 1]), None, at(b.g_all, p), None)), at(b.gz, p),
             at(b.gagg, p), at(b.G, p), at(b.sigma, p), at(b.gQ, p), at(b.ln_part, p), at(b.te_part, p), pa, po, seed,
             P(b.rng_step), p, at(b.sdrop, p), None, s), "sgl_conv_backward")
 
@@ -94,3 +95,34 @@ def test_passes_in_one_launch_equal_single_passes(gpu, D, F, T, H, k, U, edges):
     assert torch.isfinite(live).all()
     if edges:   # the passes drew their own masks
         assert not torch.equal(live[0], live[1]) and not torch.equal(live[1], live[2])
+
+
+@pytest.mark.parametrize("D,F,T,H,k,U,edges", [(100, 172, 100, 2, 10, 45, True), (172, 16, 100, 4, 20, 9, True),
+                                               (32, 6, 16, 1, 5, 16, True), (32, 6, 16, 4, 5, 16, False)])
+def test_passes_from_a_given_gradient(gpu, D, F, T, H, k, U, edges):
+    """dL/dy given (gy): every pass from it, the weight gradients pass 0's, the accumulators untouched."""
+    drop = (0.25, 0.1, 123456789)
+    got, grads = {}, {}
+    for how in ("one launch", "one at a time"):
+        step, params, feat, pred_w = _step(gpu, D, F, T, H, k, U, edges, seed=D + k + U)
+        b = step.buf
+        gy = torch.randn(b.cap, D, generator=torch.Generator().manual_seed(3)).to(gpu)
+        acc = b.acc_all.clone()
+        step.edge_rows(feat)
+        if how == "one launch":
+            step.conv_forward(params, feat, drop=drop)
+            grads[how] = step.conv_backward(params, feat, gy, drop=drop)
+        else:
+            _one_at_a_time(step, params, pred_w, drop, gy)
+            grads[how] = step._weight_grad_products(params, True, step.bwd_tile_rows(False))
+        torch.cuda.synchronize()
+        assert torch.equal(b.acc_all, acc)
+        got[how] = {n: getattr(b, n).clone() for n in SAVED + GRADS + ("y", "X", "S", "phi0", "g_all")}
+    for n, v in got["one launch"].items():
+        assert torch.equal(v, got["one at a time"][n]), n
+    # sums of at most U float32 products in two orders, each within U * 2^-24 of the sum of their magnitudes
+    for n in ("gz", "gagg", "gQ", "G", "Q", "sigma", "agg", "xbar", "new_mem", "sdrop", "ln_part", "te_part"):
+        getattr(b, n).abs_()
+    sizes = step._weight_grad_products(params, True, step.bwd_tile_rows(False))
+    for i, (x, y, m) in enumerate(zip(*grads.values(), sizes)):
+        assert bool(((x.reshape(-1) - y.reshape(-1)).abs() <= 2 * (U + 8) * 2.0 ** -24 * m.abs().reshape(-1)).all()), i
