@@ -21,6 +21,7 @@
 //   D = 100, S = 372, K = 1: 31.4 (+ 4.7 the commit) -> 10.7 + 11.3 us at 320
 //   roots; rows without messages (the updater module, 333): 30.1 ->
 //   8.9 + 10.7 us, and 85 -> 21 us with the host's part (8 fills fewer).
+#include <algorithm>
 #include <climits>
 
 #include "common.h"
@@ -35,11 +36,27 @@ constexpr int kInWaves = kInBlock / sgl::kWave;
 constexpr int kMsgParts = 2;    // workgroups of a tile's messages
 constexpr int kMaxWidth = 512;  // S = 2D + F (so D <= 256: at most 16 column chunks)
 
-// Above this capacity the one-launch kernel has a tile for most CUs and the
-// workspace's traffic is no longer free (split against one launch, us: D 100, S
-// 372, K 1: 2,048 rows 28 / 31, 4,096 35 / 32; D 172, S 360, K 4: 117 / 132 and
-// 176 / 139; D 64, S 144, K 2: 18 / 22 and 24 / 23).
-constexpr int64_t kSplitMaxRows = 2048;
+// Narrow hidden rows need few waves for their products; the messages (a root a
+// wave, a chain of loads each) then set the time. With messages at least this
+// many workgroups of a tile stage them and this many waves a workgroup write
+// them (split / one launch and the commit, us, 1,000 events: D 4, F 1, K 1
+// 21.5 -> 11.3 / 12.8; D 16, F 16, K 4 23.3 -> 17.3 / 20.0; D 32, F 172, K 1
+// 18.1 -> 15.7 / 18.6; from D 64 on the products have as many).
+constexpr unsigned kMsgGroups = 4, kMsgWaves = 4;
+constexpr unsigned kXcds = 8;
+
+// Above these capacities the one-launch kernel has a tile for most CUs and the
+// workspace's traffic is no longer free (split / one launch, us: D 100, S 372,
+// K 1: 2,048 rows 29 / 34, 4,096 35 / 32; D 172, S 360, K 4: 116 / 137 and 176 /
+// 139; D 64, S 144, K 2: 18 / 22 and 24 / 23). Rows that are not whole 16 bytes
+// load word by word, which wide products pay for earlier (D 172, S 345, K 1:
+// 1,024 rows 43 / 53, 1,280 53 / 53, 2,048 61 / 54), as do a partial column
+// block and more than 12 waves (D 200, S 400, K 2: 1,024 rows 86 / 93, 2,048
+// 103 / 95; D 192 94 / 112, D 240 133 / 155).
+int64_t split_max_rows(int D, int F) {
+  const bool words = D % 4 != 0 || F % 4 != 0;
+  return (D > 128 && words) || (D > 192 && D % 16 != 0) ? 1024 : 2048;
+}
 
 struct Events {  // one batch's messages (all NULL: none are written)
   const int64_t *src, *dst;
@@ -128,6 +145,7 @@ __global__ __launch_bounds__(kInBlock) void k_gru_inputs(
     }
     return;
   }
+  if (16 * int(blockIdx.z) * kInWaves >= G) return;  // launched for the messages only
   // the tile's rows (a row's id is read by its own lanes: one barrier fewer)
   auto row_of = [&](int i) {
     const int64_t root = roots != nullptr ? roots[r0 + i] : int64_t(r0 + i);
@@ -196,8 +214,9 @@ __device__ __forceinline__ void gates3(const float *hs, int ldh, const GateWeigh
   for (int t = 0; t < 3; ++t) acc[t] = p[t] + r[t];
 }
 
-// Grid: (tiles, 1 + message parts), one wave per 16 hidden columns (TH: their
-// most threads; fewer leave a lane more registers). A lane's loads
+// Grid: (tiles, 1 + message parts), one wave per 16 hidden columns and with
+// messages at least kMsgWaves (TH: their most threads; fewer leave a lane more
+// registers). A lane's loads
 // take clamped rows and columns instead of branches, so that all of them are
 // in flight together.
 template <int TH>
@@ -255,6 +274,14 @@ __global__ __launch_bounds__(TH) void k_gru_cells(
 
   // this lane's column and its four rows of the tile
   const int n0 = 16 * wave, col = n0 + (lane & 15), i0 = 4 * (lane >> 4);
+  if (n0 >= D) {  // a wave launched for the messages only: this workgroup's barriers
+    for (int k = 1; k < K; ++k) {
+      __syncthreads();
+      __syncthreads();
+    }
+    __syncthreads();
+    return;
+  }
   const bool cok = col < D;
   const int cc = min(col, D - 1);
   const int ldh = sgl::lds_ld(D);
@@ -330,9 +357,12 @@ int launch_split(int D, int K, int F, int64_t capacity, const int32_t *num_roots
                  const float *w_hh, const float *b_ih, const float *b_hh, const float *wc_ih, const float *wc_hh,
                  const float *bc_ih, const float *bc_hh, const Events &ev, const Commit &cm, float *new_mem, float *ws,
                  hipStream_t stream) {
-  const unsigned tiles = unsigned((capacity + kRows - 1) / kRows);
-  const unsigned groups = unsigned(((3 * D + 15) / 16 + kInWaves - 1) / kInWaves);
+  // (a multiple of the XCDs, to which workgroups are dealt in turn: a tile's
+  // workgroups of both launches share an L2, where the first leaves what the
+  // second reads)
+  const unsigned tiles = unsigned((capacity + kRows * kXcds - 1) / (kRows * kXcds) * kXcds);
   const bool msgs = ev.win_src != nullptr;
+  const unsigned groups = std::max(unsigned(((3 * D + 15) / 16 + kInWaves - 1) / kInWaves), msgs ? kMsgGroups : 1u);
   float *staged = ws + padded_rows(capacity) * size_t(K + 1) * size_t(3 * D);
   // an op timed by the caller: from the first launch's start to the second's end
   const sgl::LaunchTimer timed = sgl::pending_timer();
@@ -343,7 +373,7 @@ int launch_split(int D, int K, int F, int64_t capacity, const int32_t *num_roots
               static_cast<const int32_t *>(next_mail_pos), ws, staged);
   SGL_CHECK_LAUNCH();
   sgl::pending_timer() = sgl::LaunchTimer{nullptr, timed.stop};
-  const unsigned waves = unsigned((D + 15) / 16);
+  const unsigned waves = std::max(unsigned((D + 15) / 16), msgs ? kMsgWaves : 1u);
   const size_t lds_h = sizeof(float) * kRows * size_t(sgl::lds_ld(D));
   const auto cells = waves <= 8 ? &k_gru_cells<512> : waves <= 12 ? &k_gru_cells<768> : &k_gru_cells<1024>;
   sgl::launch(cells, dim3(tiles, msgs ? 1 + kMsgParts : 1), dim3(waves * sgl::kWave), lds_h, stream, D, K, F, num_roots,
@@ -357,7 +387,7 @@ int launch_split(int D, int K, int F, int64_t capacity, const int32_t *num_roots
 }  // namespace
 
 extern "C" size_t sgl_memory_update_workspace_bytes(int32_t D, int32_t K, int32_t F, int64_t capacity) {
-  if (D <= 0 || K <= 0 || F < 0 || capacity <= 0 || capacity > kSplitMaxRows || 2 * D + F > kMaxWidth) return 0;
+  if (D <= 0 || K <= 0 || F < 0 || capacity <= 0 || 2 * D + F > kMaxWidth || capacity > split_max_rows(D, F)) return 0;
   if (sgl_memory_update_lds_bytes(D, F) > 160 * 1024) return 0;  // shapes that sgl_memory_update refuses stay refused
   return ws_bytes(D, K, F, capacity);
 }

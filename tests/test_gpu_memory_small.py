@@ -60,6 +60,21 @@ def test_update_and_commit_equals_the_two_calls(gpu, D, F, K, B, N):
         assert torch.equal(a, b), i
 
 
+@pytest.mark.parametrize("D,F,K,B,N", [(4, 1, 3, 100, 150), (15, 172, 1, 90, 400), (33, 171, 2, 64, 90), (48, 16, 4, 70, 300),
+                                       (49, 0, 2, 129, 2000)])
+def test_narrow_rows_equal_the_two_calls(gpu, D, F, K, B, N):
+    """Fewer column blocks than the messages have waves and workgroups (four of each): the waves between."""
+    test_update_and_commit_equals_the_two_calls(gpu, D, F, K, B, N)
+
+
+def test_rows_where_one_launch_takes_over(gpu):
+    from starry_unigraph.lib import _capi
+    ws = _capi.lib().sgl_memory_update_workspace_bytes
+    for D, F, most in ((100, 172, 2048), (128, 1, 2048), (130, 0, 1024), (172, 16, 2048), (172, 1, 1024), (200, 0, 1024),
+                       (192, 4, 2048), (240, 16, 2048), (250, 0, 1024)):
+        assert ws(D, 2, F, most) > 0 and ws(D, 2, F, most + 1) == 0, (D, F)
+
+
 @pytest.mark.parametrize("M,D,F,K", [(1, 100, 172, 1), (16, 32, 0, 3), (333, 100, 172, 2), (2048, 64, 16, 4),
                                      (2049, 64, 16, 4), (47, 172, 16, 4), (20, 250, 1, 1)])
 def test_updater_rows(gpu, M, D, F, K):
