@@ -476,7 +476,10 @@ class CTDGOnlineRuntime:
             if self.plan_timer is not None:   # (entry point name, callback giving this step's event pair or None)
                 evs = self.plan_timer[1]()
                 if evs is not None:
-                    top = plan[3].index(self.plan_timer[0])
+                    names, name = plan[3], self.plan_timer[0]
+                    if name == "sgl_memory_commit" and name not in names:   # in the update's launches
+                        name = "sgl_memory_update"
+                    top = names.index(name)
                     t0, t1 = evs[0].cuda_event, evs[1].cuda_event
             _capi.check(_capi.lib().sgl_plan_run(
                 plan[0], plan[1], plan[2], front.cuda_stream, _capi.stream_of(self.device),

@@ -477,15 +477,19 @@ class DeviceStep:
             st.D, b.cap, P(b.num_roots), P(b.roots), P(b.new_mem), P(st.memory), P(st.memory_ts), P(b.ts_max),
             P(st.node_bits), P(b.hop.cnt), P(b.any_edges), P(b.root_dt), self._s()), "sgl_memory_commit"))
 
+    def commits_in_update(self, gru: dict) -> bool:
+        """Whether update_and_commit() has the commit in the update's launches
+        (timed as "memory_update", no "memory_commit")."""
+        return gru["w_ih"].dtype != torch.bfloat16 and self._gru_workspace() is not None
+
     def update_and_commit(self, gru: dict, src, dst, efeat, ts, from_cursor: bool = False) -> None:
         """update_memory() then commit(); small fp32 batches by
         sgl_memory_update_commit (the same results)."""
-        ws = None if gru["w_ih"].dtype == torch.bfloat16 else self._gru_workspace()
-        if ws is None:
+        if not self.commits_in_update(gru):
             self.update_memory(gru, src, dst, efeat, ts, from_cursor=from_cursor)
             self.commit()
             return
-        b, st, P = self.buf, self.state, _capi.ptr
+        b, st, P, ws = self.buf, self.state, _capi.ptr, self._gru_workspace()
         self._call("memory_update", lambda: _capi.check(_capi.call("sgl_memory_update_commit",
             st.D, st.K, st.F, b.cap, P(b.num_roots), P(b.roots), P(st.memory), P(st.mailbox), P(st.mailbox_ts),
             P(st.next_mail_pos), P(gru["w_ih"]), P(gru["w_hh"]), P(gru["b_ih"]), P(gru["b_hh"]), P(gru["wc_ih"]),
