@@ -1,9 +1,10 @@
 """Several dropout passes of the attention in one launch
 (sgl_conv_forward_passes / sgl_conv_backward_passes, the src, dst and negative
 roles of runtime.py:193-195) against the same passes launched one at a time:
-bit-identical outputs, saved state and gradients, for 8-wave tiles, 16-wave
-tiles with the time encodings staged in LDS and without, a partial last tile,
-a single root and a block without edges."""
+bit-identical outputs, saved state and gradients, for 8-wave tiles of 8 and of
+4 roots (two window slices each), 16-wave tiles with the heads split over the
+waves, with the time encodings staged in LDS and without, a partial last tile, a
+single root and a block without edges."""
 import pytest
 import torch
 
@@ -70,7 +71,10 @@ def _one_at_a_time(step, params, pred_w, drop, gy=None):
 
 
 @pytest.mark.parametrize("D,F,T,H,k,U,edges", [
-    (100, 172, 100, 2, 10, 45, True),    # 8 waves
+    (100, 172, 100, 2, 10, 45, True),    # 16 waves, the heads split over them
+    (128, 172, 100, 2, 10, 45, True),    # the same forward, a backward of 8 waves and 4 roots
+    (24, 332, 100, 3, 10, 29, True),     # 8 waves and 4 roots both ways
+    (24, 332, 100, 4, 9, 21, True),      # 8 waves, 8 roots, 8 column blocks
     (32, 6, 16, 2, 10, 37, True),        # 16 waves, encodings staged
     (100, 16, 100, 2, 64, 21, True),     # 16 waves, 4 * 64 * 100 encodings do not fit in LDS
     (172, 16, 100, 4, 20, 9, True),      # 8 roots a workgroup

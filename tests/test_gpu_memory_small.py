@@ -100,3 +100,18 @@ def test_updater_rows(gpu, M, D, F, K):
     want = cell(h, mem.double(), "memory_cell")
     assert out.shape == (M, D) and torch.equal(mail, before)
     assert float((out.double() - want).abs().max()) < 2e-5
+
+
+@pytest.mark.parametrize("M,D,F,K", [(1, 100, 172, 1), (16, 32, 0, 3), (333, 100, 172, 2), (47, 17, 3, 4), (1024, 250, 1, 1)])
+def test_updater_rows_equal_the_one_launch(gpu, monkeypatch, M, D, F, K):
+    """The same rows through sgl_memory_update and an identity root list (the module's way for more rows): the same bits."""
+    from starry_unigraph.backends.ctdg.runtime.models import CTDGMemoryUpdater
+    from starry_unigraph.lib import _capi
+    torch.manual_seed(M + D)
+    u = CTDGMemoryUpdater(D, 2 * D + F, K).to(gpu)
+    mail, mem = torch.randn(M, K, 2 * D + F, device=gpu), torch.randn(M, D, device=gpu)
+    assert _capi.lib().sgl_memory_update_workspace_bytes(D, K, F, M) > 0
+    out = u(mail, mem)
+    monkeypatch.setattr(_capi.lib(), "sgl_memory_update_workspace_bytes", lambda *a: 0)
+    monkeypatch.setattr(_capi.lib(), "sgl_memory_rows", None)   # (not reached)
+    assert torch.equal(out, u(mail, mem))
