@@ -10,6 +10,7 @@
 //   m = lerp(m, g, 1-b1); v = b2*v + (1-b2)*g*g;
 //   p -= (lr / (1-b1^t)) * m / (sqrt(v) / sqrt(1-b2^t) + eps)
 #include <cmath>
+#include <type_traits>
 
 #include "common.h"
 #include "mfma.h"
@@ -89,6 +90,7 @@ namespace {
 
 constexpr int kGaBlock = 256;
 constexpr int kGaChunk = 16;  // MFMA row groups per wave per load batch
+constexpr int kGaRun = 4;     // of them per sum in fp32, without ADAM
 constexpr int kGaRound = 4 * 4 * kGaChunk;  // rows of the four waves' load batches
 // Floats of a strided operand addressed from one base: with the rows that the
 // last round reads past them (masked by the range) below 2^30, 4 GiB of bytes,
@@ -142,6 +144,11 @@ __device__ __forceinline__ int job_rows(const sgl_grad_job &jb, const int32_t *n
 // 12 gradients in one launch of 4.1 us at 164 roots of 372 columns, where
 // matrix products, column sums and concatenations took 20 launches, 145 us and
 // a host read of the root count (the module's pass: 383 -> 214 us).
+// Its sums are of fp32 runs of 16 rows added in double (as a tensor's column
+// sum adds in many short runs; one fp32 chain a wave was 4 to 20 times further
+// off above 2,048 rows): 6e-8 to 1e-7 from the 64-bit gradient at 64 to 524,288
+// rows, and the shorter chains are no slower (8,192 rows of 372 columns 104 ->
+// 102 us, 65,536 1,270 -> 1,217).
 template <bool ADAM>
 __global__ __launch_bounds__(kGaBlock) void k_grad_adam(const sgl_grad_job *__restrict__ jobs,
                                                        const int32_t *__restrict__ tile_job,
@@ -150,7 +157,8 @@ __global__ __launch_bounds__(kGaBlock) void k_grad_adam(const sgl_grad_job *__re
                                                        float *__restrict__ v, AdamSegs segs,
                                                        const float *__restrict__ coef, float b1, float b2, float eps,
                                                        float wd, uint16_t *__restrict__ shadow) {
-  __shared__ float red[4][16][17];
+  using Sum = std::conditional_t<ADAM, float, double>;
+  __shared__ Sum red[4][16][17];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   sgl_grad_job jb;
   int local;
@@ -186,6 +194,7 @@ __global__ __launch_bounds__(kGaBlock) void k_grad_adam(const sgl_grad_job *__re
     const int R = job_rows(jb, num_roots);
     const int i16 = lane & 15, q = lane >> 4;
     sgl::f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    double sum[4] = {0.0, 0.0, 0.0, 0.0};
     const int npass = jb.npass > 0 ? jb.npass : 1;
     // Buffer offsets are 32-bit bytes: rows that reach further are taken in
     // segments, each from its own base, of whole rounds of the four waves
@@ -213,14 +222,23 @@ __global__ __launch_bounds__(kGaBlock) void k_grad_adam(const sgl_grad_job *__re
             xb[c] = sgl::buf_load(r2, r * uint32_t(jb.s2) + uint32_t(b0 + i16));
           }
 #pragma unroll
-          for (int c = 0; c < kGaChunk; ++c) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[c], xb[c], acc, 0, 0, 0);
+          for (int c0 = 0; c0 < kGaChunk; c0 += kGaRun) {
+            if constexpr (!ADAM) acc = sgl::f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int c = c0; c < c0 + kGaRun; ++c)
+              acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[c], xb[c], acc, 0, 0, 0);
+            if constexpr (!ADAM) {
+#pragma unroll
+              for (int e = 0; e < 4; ++e) sum[e] += double(acc[e]);
+            }
+          }
         }
       }
     }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) red[wave][4 * (lane >> 4) + e][lane & 15] = acc[e];
+    for (int e = 0; e < 4; ++e) red[wave][4 * (lane >> 4) + e][lane & 15] = ADAM ? Sum(acc[e]) : Sum(sum[e]);
     __syncthreads();
-    gv = red[0][oa][ob] + red[1][oa][ob] + red[2][oa][ob] + red[3][oa][ob];
+    gv = float(red[0][oa][ob] + red[1][oa][ob] + red[2][oa][ob] + red[3][oa][ob]);
     if (valid) g[idx] = gv;
     if constexpr (!ADAM) return;
   } else {

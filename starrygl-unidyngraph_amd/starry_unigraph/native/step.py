@@ -8,6 +8,8 @@ backends/ctdg/runtime/runtime.py:225-297):
   sgl_recent_sample   hop-0 recent-k windows of the roots          (sampler.py:93-128)
   sgl_memory_update   GRU over mailbox + memory, mailbox write     (runtime.py:268-282)
   sgl_memory_commit   memory/memory_ts scatter                     (memory.py:254-269)
+  (small fp32 batches: sgl_memory_update_commit for the two; with dropout the
+  attention's several passes by sgl_conv_forward_passes / _backward_passes)
   sgl_conv_forward    time encoding + temporal attention           (models.py:77-137)
   sgl_predictor       edge predictor + BCE, per-root gradient sums (models.py:313-324, runtime.py:290-292)
   sgl_conv_backward   attention backward                           (loss.backward(), runtime.py:296)
@@ -711,9 +713,9 @@ def weight_grads_in_one_launch(rows: int, D: int, C: int) -> bool:
     a 16x16 block, and each strip of X is read by D / 16 of them, so rows x D x
     C sets its time, where a matrix product splits the rows. One launch against
     products, us, at 8,192 / 65,536 / 131,072 rows: D 100, C 372, two heads
-    104 / 390, 1,279 / 1,748, 2,927 / 2,728; D 172, C 288, four heads 185 / 407,
+    102 / 390, 1,217 / 1,748, 2,927 / 2,728; D 172, C 288, four heads 184 / 407,
     1,980 / 1,975, 4,332 / 3,032 (the two meet at 65,536: 3.2e9); D 64, C 120,
-    four heads 44 / 391, 380 / 1,188, 755 / 2,166."""
+    four heads 39 / 391, 310 / 1,181, 622 / 2,165."""
     return rows * D * C <= GRAD_LAUNCH_MAX
 
 

@@ -104,3 +104,24 @@ def test_rows_past_32_bit_offsets(gpu, R, s1, s2):
     assert torch.equal(*got)
     size = x[0].abs().double().T @ x[1].abs().double()
     assert bool(((got[0].double() - x[0].double().T @ x[1].double()).abs() <= (R + 8) * 2.0 ** -24 * size).all())
+
+
+@pytest.mark.parametrize("R", [300, 8192, 100003])
+def test_long_sums_keep_their_precision(gpu, R):
+    """Against float64: half a unit of the result's last place and runs of 16 rows rounded independently, together about
+    1e-7 of the result's norm at any length (one float32 chain a wave is at 8e-7 at 8,192 rows, 2e-6 at 65,536)."""
+    from starry_unigraph.lib import _capi
+    g = torch.Generator().manual_seed(R)
+    x1, x2, one = torch.randn(R, 48, generator=g).to(gpu), torch.randn(R, 33, generator=g).to(gpu), torch.ones(1, device=gpu)
+    jobs = (_capi.GradJob * 2)(
+        _capi.GradJob(x1=x1.data_ptr(), x2=x2.data_ptr(), s1=48, s2=33, off=0, ldo=33, rows=48, cols=33, kind=0, r_fixed=-1,
+                      tiles_b=3, npass=1),
+        _capi.GradJob(x1=x1.data_ptr(), x2=one.data_ptr(), s1=48, s2=0, off=48 * 33, ldo=1, rows=48, cols=1, kind=0,
+                      r_fixed=-1, tiles_b=1, npass=1))
+    raw = torch.frombuffer(bytearray(bytes(jobs)), dtype=torch.uint8).to(gpu)
+    tiles = torch.tensor([256 * i for i in range(9)] + [256 * i + 1 for i in range(3)], dtype=torch.int32, device=gpu)
+    n, out = torch.tensor([R], dtype=torch.int32, device=gpu), torch.empty(48 * 34, device=gpu)
+    _capi.check(_capi.lib().sgl_weight_grads(raw.data_ptr(), tiles.data_ptr(), 12, n.data_ptr(), out.data_ptr(),
+                                             _capi.stream_of(gpu)), "sgl_weight_grads")
+    for got, want in ((out[:48 * 33].view(48, 33), x1.double().T @ x2.double()), (out[48 * 33:], x1.double().sum(0))):
+        assert float((got.double() - want).norm() / want.norm()) < 2e-7
