@@ -18,9 +18,9 @@
 // writes the memory table (the commit's launch is saved) and, by its other
 // workgroups, the staged messages. Per value the same products in the same
 // order as k_gru_mailbox: the same bits.
-//   D = 100, S = 372, K = 1: 31.4 (+ 4.7 the commit) -> 10.7 + 11.3 us at 320
+//   D = 100, S = 372, K = 1: 31.4 (+ 4.7 the commit) -> 9.6 + 11.6 us at 320
 //   roots; rows without messages (the updater module, 333): 30.1 ->
-//   8.9 + 10.7 us, and 85 -> 21 us with the host's part (8 fills fewer).
+//   8.1 + 11.0 us, and 85 -> 21 us with the host's part (8 fills fewer).
 #include <algorithm>
 #include <climits>
 

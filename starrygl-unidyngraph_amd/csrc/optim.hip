@@ -141,7 +141,7 @@ __device__ __forceinline__ int job_rows(const sgl_grad_job &jb, const int32_t *n
 
 // ADAM false: the gradients alone (p, m, v, coef and the gates unused; kind-1
 // jobs have nothing to do). For the attention module's autograd backward:
-// 12 gradients in one launch of 4.1 us at 164 roots of 372 columns, where
+// 12 gradients in one launch of 4.4 us at 164 roots of 372 columns, where
 // matrix products, column sums and concatenations took 20 launches, 145 us and
 // a host read of the root count (the module's pass: 383 -> 214 us).
 // Its sums are of fp32 runs of 16 rows added in double (as a tensor's column

@@ -407,8 +407,9 @@ __global__ __launch_bounds__(kPrepBlock) void k_step_prepare_wg(
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   if (gate_word != nullptr) {
     // a launch plan's cross-stream gate, before anything is read or written:
-    // thread 0's acquire loads invalidate this CU's L1 and the XCD's L2 for
-    // the whole workgroup (one CU), which the barrier then orders after
+    // the acquire fence at the end of thread 0's wait invalidates this CU's L1
+    // and the XCD's L2 for the whole workgroup (one CU), which the barrier then
+    // orders after
     if (tid == 0) sgl::gate_wait(gate_word, gate_value, gate_timeout);
     __syncthreads();
   }
