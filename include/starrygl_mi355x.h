@@ -128,7 +128,7 @@ int sgl_recent_sample_packed(const int64_t *indptr, const int32_t *nbr_eid,
  * build's sampler): nbr_eid [num_edges][2], ts32 [num_edges], fence
  * [ceil(num_edges / 32)], and in flags (two int64, zero on entry) whether
  * they may be used: flags[1] != 0: some timestamp does not fit in int32
- * (use none of them); flags[0] != 0: some node's list is not sorted by time
+ * (use none of them, nor flags[0]); flags[0] != 0: some node's list is not sorted by time
  * (pass no fence). */
 int sgl_recent_pack(int64_t num_nodes, int64_t num_edges, const int64_t *indptr,
                     const int32_t *nbr, const int32_t *eid, const int64_t *ts,

@@ -122,7 +122,9 @@ __global__ __launch_bounds__(kBlock) void k_tcsr_indptr(int64_t num_nodes, int64
 // bound by the bytes (28 per edge). Tensor operations for the same (two
 // reductions, a stack, and a sort-based lookup of the decreasing places among
 // the list starts) took about 900 us at 7.8 M edges and 1.1 M nodes, this 61
-// (219 MB: 3.6 TB/s).
+// (219 MB: 3.6 TB/s). A thread that meets a time outside int32 stops: a graph
+// of such times is told in 61 us at 20 M edges (103 by two reductions, 192
+// with its copy written).
 constexpr int64_t kFenceSpan = 32;
 __global__ __launch_bounds__(kBlock) void k_recent_pack(
     int64_t num_edges, int64_t num_nodes, const int64_t *__restrict__ indptr, const int32_t *__restrict__ nbr,
@@ -134,14 +136,16 @@ __global__ __launch_bounds__(kBlock) void k_recent_pack(
   for (int64_t i = first; i < num_edges; i += step) {
     const int64_t t = ts[i];
     const int64_t before = i > 0 ? ts[i - 1] : t;  // (the neighbouring lane's line)
-    nbr_eid[i] = make_int2(nbr[i], eid[i]);
+    const int2 ids = make_int2(nbr[i], eid[i]);
+    wide = t != int64_t(int32_t(t));
+    if (wide) break;  // nothing of the copy is used
+    nbr_eid[i] = ids;
     ts32[i] = int32_t(t);
     if (i % kFenceSpan == 0) fence[i / kFenceSpan] = int32_t(t);
-    wide |= t != int64_t(int32_t(t));
     down += t < before;
   }
   // list starts (the entries past the last list, if any, form one more)
-  for (int64_t n = first; n <= num_nodes; n += step) {
+  for (int64_t n = first; n <= num_nodes && !wide; n += step) {
     const int64_t s = indptr[n], e = n < num_nodes ? indptr[n + 1] : num_edges;
     if (s > 0 && s < e) down -= ts[s] < ts[s - 1];
   }
