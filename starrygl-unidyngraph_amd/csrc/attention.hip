@@ -376,9 +376,11 @@ __global__ __launch_bounds__(NW * 64) void k_conv_fwd(
   const unsigned long long dstep = DROP ? *dc.step : 0ull;
   const float sa = sgl::drop_scale(dc.p_att), so = sgl::drop_scale(dc.p_out);
   if constexpr (DROP) {  // grid row p: dropout pass dc.pass + p, its own masks, saved state and output
-    to_pass(sv, d, size_t(gridDim.x) * RPW, blockIdx.y);
-    y += blockIdx.y * y_pass_stride;
-    dc.pass += blockIdx.y;
+    if (blockIdx.y > 0) {
+      to_pass(sv, d, size_t(gridDim.x) * RPW, blockIdx.y);
+      y += blockIdx.y * y_pass_stride;
+      dc.pass += blockIdx.y;
+    }
   }
   if (nrows == 0 || !live) {
     // rows outside the live set: zero output (y's row U is the null
@@ -1464,8 +1466,29 @@ struct BwdPickDropWide {
 //   B = 600, 432 columns, 2 heads, 20 entries: 60.2 -> 47.5 / (45.4: spills)
 //   B = 200 / 3000, 120 columns, 4 heads:     23.1 -> 22.0, 24.4 -> 23.3 / 21.8 -> 20.9, 22.8 -> 22.4
 //   B = 600 / 3000, 216 columns, 4 heads:     37.2 -> 30.4, 46.9 -> 37.6 / 31.6 -> 27.0, 38.7 -> 33.1
+// (few live roots a batch.) It does not pay everywhere, 8 waves -> split, us,
+// 1,200 roots if not said otherwise (one pass with dropout):
+//   - up to 128 columns 8 waves leave room for two workgroups a CU: backward,
+//     120 columns, 4 heads, 12,000 roots of 10 entries 154 -> 266; the forward
+//     gains from windows of 16 on (5 entries 39 -> 39, 20 52 -> 48, 64 88 -> 79);
+//   - with dropout both waves of a root draw each entry's masks: forward, 372
+//     columns, 2 heads, 10 entries 75 -> 70, 64 130 -> 130, 200 284 -> 307; 216
+//     columns, 4 heads, 20 entries 96 -> 83, 64 164 -> 151, 400 715 -> 707; 168
+//     columns, 20 entries 68 -> 67, 64 115 -> 122; backward, 216 columns, 20 entries 87 -> 82, 64
+//     147 -> 144, 12,000 roots of 64 874 -> 909; 168 columns, 10 entries 55 -> 56;
+//     372 columns, 10 entries 73 -> 71, 20 82 -> 81, 64 116 -> 119; 340, 10 64 -> 65;
+//   - backward, 260 columns, 2 heads, 10 entries 47 -> 48 (300 columns 61 -> 58).
 constexpr bool split_fp32(int hm, int jm) { return split_heads(hm, jm) && hm * jm <= 24; }
-constexpr bool split_fp32_bwd(int hm, int jm) { return split_heads(hm, jm) && jm <= 6 && hm * jm <= 16; }
+constexpr bool split_fp32_bwd(int hm, int jm, bool drop) {
+  return split_heads(hm, jm) && jm >= 4 && jm <= (drop ? 4 : 6) && hm * jm <= 16;
+}
+inline bool split_fwd_pays(const Dims &d, bool drop) {
+  if (d.C <= 128) return !drop && d.k >= 16;
+  return !drop || d.k <= (d.C > 192 && d.C <= 256 ? 64 : 20);
+}
+inline bool split_bwd_pays(const Dims &d, bool drop) {
+  return drop ? d.C > 192 && d.k <= 20 : d.C <= 256 || d.C > 280;
+}
 template <bool DROP>
 struct Split {
   template <int HM, int JM>
@@ -1478,7 +1501,7 @@ struct Split {
   template <int HM, int JM>
   struct Bwd {
     static Instance<BwdFn> get() {
-      if constexpr (split_fp32_bwd(HM, JM)) return {&k_conv_bwd<HM, JM, DROP, false, 16, kFp32Rows, 2>, 16, kFp32Rows, 2};
+      if constexpr (split_fp32_bwd(HM, JM, DROP)) return {&k_conv_bwd<HM, JM, DROP, false, 16, kFp32Rows, 2>, 16, kFp32Rows, 2};
       else return {nullptr, 0, 0};
     }
   };
@@ -1505,12 +1528,13 @@ bool fp32_four_fits(const Dims &d, int nw) {
          sizeof(float) * bwd_lds_floats(d, nw, kFp32Rows, slices) <= 160 * 1024;
 }
 // The instance that runs: `four`, or its twin `split` with the same rows (so
-// the caller's per-tile arrays stay as they are) where there is one and its
-// larger layout fits, or `wide`.
+// the caller's per-tile arrays stay as they are) where there is one, it pays
+// and its larger layout fits, or `wide`.
 template <class Fn>
-Instance<Fn> fp32_or_wide(const Dims &d, Instance<Fn> four, Instance<Fn> (*wide)(const Dims &), Instance<Fn> split) {
+Instance<Fn> fp32_or_wide(const Dims &d, Instance<Fn> four, Instance<Fn> (*wide)(const Dims &), Instance<Fn> split,
+                          bool split_pays) {
   if (four.fn != nullptr && !fp32_four_fits(d, four.waves)) return wide(d);
-  return split.fn != nullptr && lds_bytes(d, split) <= kLdsBytes ? split : four;
+  return split_pays && split.fn != nullptr && lds_bytes(d, split) <= kLdsBytes ? split : four;
 }
 
 // The bf16 weight copies' shapes (sgl_bf16_weights): every pointer set,
@@ -1591,8 +1615,7 @@ extern "C" int sgl_dropout_masks(int64_t rows, int32_t fanout, int32_t H, int32_
 extern "C" int32_t sgl_conv_tile_rows(int32_t D, int32_t F, int32_t T, int32_t H) {
   const Dims d{D, F, T, H, D + F + T, H > 0 ? D / H : 0, 0};
   if (check_dims(d) != SGL_OK) return 0;
-  const auto inst = fp32_or_wide(d, pick_instance<BwdPick>(d), &pick_instance<BwdPickWide>,
-                                      pick_instance<Split<false>::Bwd>(d));
+  const auto inst = fp32_or_wide(d, pick_instance<BwdPick>(d), &pick_instance<BwdPickWide>, Instance<BwdFn>{nullptr, 0, 0}, false);
   return inst.fn != nullptr ? inst.rows : 0;
 }
 
@@ -1600,8 +1623,8 @@ extern "C" int32_t sgl_conv_backward_tile_rows(int32_t D, int32_t F, int32_t T, 
   const Dims d{D, F, T, H, D + F + T, H > 0 ? D / H : 0, 0};
   if (check_dims(d) != SGL_OK) return 0;
   const auto inst = bf16 ? pick_instance<BwdPickBf>(d)
-                         : fp32_or_wide(d, pick_instance<BwdPick>(d), &pick_instance<BwdPickWide>,
-                                      pick_instance<Split<false>::Bwd>(d));
+                         : fp32_or_wide(d, pick_instance<BwdPick>(d), &pick_instance<BwdPickWide>, Instance<BwdFn>{nullptr, 0, 0},
+                                        false);
   return inst.fn != nullptr ? inst.rows : 0;
 }
 
@@ -1659,9 +1682,9 @@ extern "C" int sgl_conv_forward_passes(int32_t D, int32_t F, int32_t T, int32_t 
               "conv_forward: NULL array");
   const auto inst = bw != nullptr ? pick_instance<FwdPickBf>(d)
                     : drop ? fp32_or_wide(d, pick_instance<FwdPickDrop>(d), &pick_instance<FwdPickDropWide>,
-                                      pick_instance<Split<true>::Fwd>(d))
+                                        pick_instance<Split<true>::Fwd>(d), split_fwd_pays(d, true))
                            : fp32_or_wide(d, pick_instance<FwdPick>(d), &pick_instance<FwdPickWide>,
-                                      pick_instance<Split<false>::Fwd>(d));
+                                        pick_instance<Split<false>::Fwd>(d), split_fwd_pays(d, false));
   SGL_REQUIRE(inst.fn != nullptr, "conv_forward: no kernel instance for H=%d C=%d", H, d.C);
   // stage the tile's time encodings in LDS when they fit
   int ts_rows = fanout > 0 && T > 0 ? inst.rows * fanout : 0;
@@ -1714,9 +1737,9 @@ extern "C" int sgl_conv_backward_passes(int32_t D, int32_t F, int32_t T, int32_t
               "conv_backward: NULL array");
   const auto inst = bw != nullptr ? pick_instance<BwdPickBf>(d)
                     : drop ? fp32_or_wide(d, pick_instance<BwdPickDrop>(d), &pick_instance<BwdPickDropWide>,
-                                      pick_instance<Split<true>::Bwd>(d))
+                                        pick_instance<Split<true>::Bwd>(d), split_bwd_pays(d, true))
                            : fp32_or_wide(d, pick_instance<BwdPick>(d), &pick_instance<BwdPickWide>,
-                                      pick_instance<Split<false>::Bwd>(d));
+                                        pick_instance<Split<false>::Bwd>(d), split_bwd_pays(d, false));
   SGL_REQUIRE(inst.fn != nullptr, "conv_backward: no kernel instance for H=%d C=%d", H, d.C);
   // one ln_part / te_part tile per workgroup: the caller sized them by
   // sgl_conv_backward_tile_rows (the dropout instances' rows are the fp32 ones)

@@ -71,8 +71,8 @@ def _one_at_a_time(step, params, pred_w, drop, gy=None):
 
 
 @pytest.mark.parametrize("D,F,T,H,k,U,edges", [
-    (100, 172, 100, 2, 10, 45, True),    # 16 waves, the heads split over them
-    (128, 172, 100, 2, 10, 45, True),    # the same forward, a backward of 8 waves and 4 roots
+    (100, 172, 100, 2, 10, 45, True),    # a forward of 16 waves, the heads split over them; a backward of 8 and 4 roots
+    (100, 16, 100, 4, 10, 21, True),     # the heads split both ways
     (24, 332, 100, 3, 10, 29, True),     # 8 waves and 4 roots both ways
     (24, 332, 100, 4, 9, 21, True),      # 8 waves, 8 roots, 8 column blocks
     (32, 6, 16, 2, 10, 37, True),        # 16 waves, encodings staged

@@ -83,3 +83,13 @@ def test_split_heads_match_float64(gpu, D, F, T, H, k, U, p):
         of = "w_v.weight" if k == 1 and n[:3] in ("w_q", "w_k") else "w_k.weight" if n == "w_k.bias" else n
         size = own[of].grad.abs().max()
         assert float((got.cpu().double().reshape(own[n].shape) - own[n].grad).abs().max()) <= tol * float(size), n
+
+
+@pytest.mark.parametrize("p", [0.0, 0.2])
+@pytest.mark.parametrize("D,F,T,H,k,U", [
+    (64, 16, 40, 4, 15, 9), (64, 16, 40, 4, 16, 21), (64, 64, 64, 4, 20, 9), (64, 65, 64, 4, 20, 13), (64, 65, 64, 4, 21, 5), (64, 64, 64, 4, 21, 5),
+    (100, 16, 100, 4, 64, 6), (100, 16, 100, 4, 65, 6), (100, 80, 100, 2, 20, 9), (100, 81, 100, 2, 21, 9)])
+def test_either_side_of_the_split(gpu, D, F, T, H, k, U, p):
+    """The widths and window lengths at which the forward or the backward goes from one instance to the other, so that
+    the two directions of a pass run different ones."""
+    test_split_heads_match_float64(gpu, D, F, T, H, k, U, p)
