@@ -69,7 +69,7 @@ constexpr int rows_for(int nw) { return nw == 16 ? 4 : 8; }
 // about what one of 8 does, and twice the workgroups share the step's roots
 // (config 1, 8 waves: forward 44.0 -> 37.8 us, backward 41.3 -> 33.9 us;
 // 2 roots 37.4 / 35.4); with several heads their 16-wave twins run where the
-// layouts fit (Split: 35.3 -> 32.3 and 31.1 -> 28.4 us). Wider shapes (config
+// layouts fit and they pay (Split: 35.3 -> 32.3 and 31.1 -> 28.4 us). Wider shapes (config
 // 5's 4 heads of 288 columns: the merge partials need 184 KB) keep 8 roots,
 // one wave each.
 constexpr int kFp32Rows = 4;

@@ -16,8 +16,9 @@ backends/ctdg/runtime/runtime.py:225-297):
   sgl_grad_adam       weight gradients + Adam, the attention segments
                       gated by "block has edges"                   (optimizer.step(), runtime.py:297)
 
-The first three are a step's front part, the memory commit its split point,
-the rest its back part (see the runtime's launch plans).
+The calls up to the memory commit, the sampled edges' rows (sgl_edge_rows) and
+the Adam step counts (sgl_adam_coef) are a step's front part, the attention and
+all after it its back part (see the runtime's launch plans).
 """
 from __future__ import annotations
 
